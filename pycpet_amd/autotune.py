@@ -109,7 +109,8 @@ def tune_grid(ctx: nat.Context, axes, x, q, *, want_phi=False, cache: Optional[d
         a, b = cache[k]
         ctx.set_tuning(0, a, b)
         return a, b
-    cands = [(kk, s) for kk in ks for s in splits]
+    # (0, 0): the library's own choice, which interpolates large grids
+    cands = [(0, 0)] + [(kk, s) for kk in ks for s in splits]
     best, _ = sweep(ctx, 0, cands,
                     lambda: ops.field_grid(*axes, x, q, want_phi=want_phi, ctx=ctx), phase=0)
     if cache is not None:
@@ -152,8 +153,9 @@ def tune_batch_volume(ctx: nat.Context, frames, *, cache: Optional[dict] = None,
         a, b = cache[k]
         ctx.set_tuning(4, a, b)
         return a, b
-    best, _ = sweep(ctx, 4, [(kk, 0) for kk in ks], lambda: B.batch_volume(frames, ctx=ctx),
-                    phase=0)
+    # (0, 0): the library's own choice, which interpolates large grids
+    best, _ = sweep(ctx, 4, [(0, 0)] + [(kk, 0) for kk in ks],
+                    lambda: B.batch_volume(frames, ctx=ctx), phase=0)
     if cache is not None:
         cache[k] = list(best)
     ctx.set_tuning(4, *best)

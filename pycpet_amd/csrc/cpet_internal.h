@@ -143,6 +143,8 @@ enum Slot : int {
   kSlotCluster2,     // cluster step: output
   kSlotNear,         // grid kernels: charge-near-grid flags
   kSlotFar,          // streamlines: far-field charge records + per-frame flags
+  kSlotFarGrid,      // interpolating grid path: node sums, weights, near lists
+  kSlotFarTables,    // its frames (written by upload_table only)
   kSlotCount
 };
 
@@ -175,6 +177,7 @@ enum TableKey : int {
   kTabPackX = 0, kTabPackC, kTabPackX2, kTabPackC2,
   kTabVolGeo, kTabVolAx, kTabVolOut, kTabVolBlk,
   kTabTopoHd, kTabTopoSl, kTabTopoAs, kTabTopoBlk,
+  kTabFarFrames,
   kTabCount
 };
 int upload_table(cpet_ctx* ctx, int key, void* dst, const void* src, size_t bytes);

@@ -1,0 +1,40 @@
+// Grid field with the far charges interpolated (fargrid.hip).
+#pragma once
+
+#include <vector>
+
+#include "cpet_internal.h"
+
+namespace cpet {
+
+// One grid of a call: axis i is n[i] values from ax0[i] on, its charges are
+// [ch0, ch0 + npad) of the packed array, its points go from out0 on.
+struct FarGrid {
+  int n[3];
+  long long ax0[3];
+  int npad;
+  long long ch0;
+  long long out0;
+};
+
+// Axes shorter than the 12 nodes by more than a third would sum at more nodes
+// than points.  The launches and node sums cost at least 60 us, which the
+// direct kernel takes at about 1e8 point-charge pairs: 41^3 x 1k (7e7 pairs)
+// 54 us direct, 41^3 x 4k (2.8e8) 150 us direct and 90 us here.  In a batch
+// the launches are shared, and the direct kernel has no charge split: a 21^3 x
+// 40k frame alone keeps it busy for 1.5 ms.
+constexpr int kFarMinAxis = 8;
+constexpr double kFarMinPairs = 2e8;
+constexpr double kFarMinPairsBatch = 2e7;
+
+// Whether an nx x ny x nz grid of npad (padded) charges takes the
+// interpolating path, from min_pairs (points x charges) on.
+bool far_grid_ok(int nx, int ny, int nz, int npad, double min_pairs);
+
+// Float32 E and / or phi of the grids (null: not wanted), queued on the
+// context's stream.  ax: the device arrays that hold the grids' x, y and z
+// axes.
+int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const float* const (&ax)[3],
+                    const float4* ch, bool want_e, bool want_phi, bool soft, void* e, void* phi);
+
+}  // namespace cpet

@@ -1,0 +1,932 @@
+// Field and potential on a box grid with the far charges interpolated.
+//
+// The direct sum over a grid costs (points x charges) pair terms, but a box
+// grid samples the smooth field of a charge a few box widths away far more
+// densely than that field varies.  Here the grid is cut into cells, halved
+// per axis level by level; a charge far from a cell contributes to the cell's
+// 12 x 12 x 12 Chebyshev nodes instead of its points, at the coarsest level
+// whose cell it is far from, and the node sums are interpolated down to the
+// points (tensor-product Lagrange).  Charges far from no cell of a point's
+// path are summed directly at the point.  All sums, nodes and interpolation
+// are FP64 (the pair terms as in the "mixed" precision: FP64 displacement and
+// r^2, FP32 rsq seed, FP64 correction), so nothing needs the FP32 error check
+// and recompute of the direct grid kernel.
+//
+// Far means that along every axis the nearest singularity of the charge's
+// field, seen from any point of the cell, lies outside the Bernstein ellipse
+// of parameter kRho = 7: the kP nodes then miss one charge's term by at most
+// 1e-9 of itself (E; 1e-10 for phi) at the threshold, and by much less beyond
+// it, against the 6e-8 rounding of one FP32 pair term.  On the frames below
+// the results are the FP64 sums rounded to float32, also where E or phi is
+// 1e-3 of its RMS (measured: within 6e-11 RMS there).  kRho = 6 was 10-15 %
+// faster and up to 1e-10 RMS off at those points, kRho = 8 10-13 % slower and
+// no nearer.
+//
+// Stages, each one launch for all frames of a call:
+//   far_classify  which charges are far from, or near, which cells: one
+//                 64-bit mask per (cell, 64 charges); and, in its last
+//                 workgroups, cell extents, Lagrange weights of every axis
+//                 value and the node transfer matrices
+//   far_nodes     node sums of every cell, split over its far charges
+//   far_reduce    the splits' partial sums in a fixed order
+//   far_eval      nodes -> points, plus the near charges, and the store
+// Every list and sum has a fixed order: results are reproducible bit for bit.
+
+#include <algorithm>
+#include <cstring>
+#include <vector>
+
+#include "cpet_internal.h"
+#include "fargrid.h"
+
+namespace cpet {
+namespace {
+
+constexpr int kP = 12;                 // nodes per axis
+constexpr int kNodes = kP * kP * kP;
+constexpr int kLeafMax = 27;           // points per axis of a leaf, at most
+constexpr int kMaxHalvings = 4;        // per axis: grids of up to 432 points
+constexpr int kMaxLevels = kMaxHalvings + 1;
+constexpr int kMaxAxis = kLeafMax << kMaxHalvings;
+constexpr int kMaxSegs = 2048;         // 64-charge segments: up to 131,072 charges
+constexpr int kThirds = 3;             // node workgroups per (cell, split)
+constexpr int kNodeLanes = 192;        // 48 node lines x 4 threads of 3 nodes
+constexpr int kNodeGroups = 4;         // that split a workgroup's charges
+constexpr int kNodeThreads = kNodeLanes * kNodeGroups;
+constexpr int kBatch = kNodeThreads;   // far charges staged per round
+constexpr int kRedThreads = 256;
+constexpr int kEvalThreads = 256;
+constexpr int kPlanes = 2;             // x planes per eval workgroup
+constexpr int kNearLds = kEvalThreads; // near charges staged at once
+
+constexpr int kGeoPerAxis = (2 << kMaxHalvings) - 1;  // intervals of all levels
+
+// Bernstein parameter kRho: sigma = (rho + 1 / rho) / 2; a charge at offset d
+// from the cell's centre (per axis) and gap g from its faces is outside the
+// ellipse of axis i when d_i^2 / sigma^2 + (|g|^2 - g_i^2) / (sigma^2 - 1)
+// >= a_i^2.
+constexpr float kRho = 7.0f;
+constexpr float kSigma = (kRho + 1.0f / kRho) / 2.0f;
+constexpr float kInvS2 = 1.0f / (kSigma * kSigma);
+constexpr float kInvS21 = 1.0f / (kSigma * kSigma - 1.0f);
+constexpr float kMinGap2 = 1e-4f;   // 0.01 A: far charges never reach the r^2 floor
+constexpr float kMaxCoord = 1e6f;   // beyond (or not finite): summed directly
+
+// cos((2k + 1) pi / 24) and (-1)^k sin((2k + 1) pi / 24): the Chebyshev nodes
+// of the first kind and their barycentric weights.
+__constant__ const double kNodeX[kP] = {
+    0.9914448613738104,  0.9238795325112867,  0.7933533402912352,  0.6087614290087207,
+    0.3826834323650898,  0.13052619222005157, -0.13052619222005157, -0.3826834323650898,
+    -0.6087614290087207, -0.7933533402912352, -0.9238795325112867, -0.9914448613738104};
+__constant__ const double kNodeW[kP] = {
+    0.13052619222005157, -0.3826834323650898, 0.6087614290087207, -0.7933533402912352,
+    0.9238795325112867,  -0.9914448613738104, 0.9914448613738104, -0.9238795325112867,
+    0.7933533402912352,  -0.6087614290087207, 0.3826834323650898, -0.13052619222005157};
+
+__host__ __device__ inline int part_begin(int n, int level, int t) { return (n * t) >> level; }
+
+// One frame of a call.  Offsets are in elements of the buffers in FarArgs.
+struct FarFrame {
+  int n[3];            // grid points per axis
+  int l[3];            // halvings per axis
+  int levels;          // max(l) + 1
+  int nseg;            // 64-charge segments
+  int cells;           // of all levels
+  int splits[kMaxLevels];
+  int xblocks;         // eval workgroups per leaf
+  int class_blk0, node_blk0, red_blk0, eval_blk0;
+  long long ch0;       // first charge
+  long long part0;     // partial node sums
+  long long val0;      // node sums of every cell, level by level
+  long long geo0;      // 3 x kGeoPerAxis x (centre, half width)
+  long long lag0[3];   // per axis: level x axis value x kP weights
+  long long tr0[3];    // per axis: leaf part x ancestor level x kP x kP
+  long long mask0;     // (cells + leaves) x nseg: far masks, then the leaves' near masks
+  long long near0;     // per leaf: number of near charges, then their numbers (64 nseg)
+  long long out0;      // first output point
+  long long ax0[3];    // first value of each axis
+};
+
+struct FarArgs {
+  int F;
+  const float* ax[3];
+  const FarFrame* frames;  // (F) when F > 1
+  FarFrame one;            // F == 1
+  const float4* ch;
+  double* part;
+  double* val;
+  double* geo;
+  double* lag;
+  unsigned long long* mask;
+  int* near;
+  void* e;
+  void* phi;
+};
+
+// A frame as kernels read it: in constant memory (the kernel's arguments or
+// the uploaded table, neither of which a kernel writes), by scalar loads.
+typedef const __attribute__((address_space(4))) FarFrame Frame;
+
+template <class Fr>
+__host__ __device__ inline int axis_level(const Fr& f, int axis, int level) {
+  return level < f.l[axis] ? level : f.l[axis];
+}
+
+template <class Fr>
+__host__ __device__ inline int cells_at(const Fr& f, int level) {
+  return 1 << (axis_level(f, 0, level) + axis_level(f, 1, level) + axis_level(f, 2, level));
+}
+
+// Parts (tx, ty, tz) of cell number c at a level (z fastest).
+__device__ __forceinline__ void cell_parts(Frame& f, int level, int c, int (&t)[3]) {
+  const int ly = axis_level(f, 1, level), lz = axis_level(f, 2, level);
+  t[2] = c & ((1 << lz) - 1);
+  t[1] = (c >> lz) & ((1 << ly) - 1);
+  t[0] = c >> (lz + ly);
+}
+
+// Number of the cell at `level` that holds the cell (t) of a deeper level.
+__device__ __forceinline__ int ancestor(Frame& f, int level, int deep, const int (&t)[3]) {
+  int c = 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int al = axis_level(f, i, level);
+    c = (c << al) | (t[i] >> (axis_level(f, i, deep) - al));
+  }
+  return c;
+}
+
+// The frame that block b belongs to.  A is the kernels' only argument.
+__device__ __forceinline__ Frame& frame_of_block(int FarFrame::*first, int b) {
+  typedef const __attribute__((address_space(4))) FarArgs Args;
+  Args* a = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+  if (a->F == 1) return a->one;
+  Frame* frames = (Frame*)(unsigned long long)a->frames;
+  int lo = 0, hi = a->F - 1;  // the last frame whose first block is <= b
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (frames[mid].*first <= b)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  return frames[lo];
+}
+
+// Lagrange weights of the kP nodes at t (barycentric, exact at a node); 0 in
+// an interval that no charge is far from, where t is not a number.
+__device__ __forceinline__ void lagrange(double t, double* __restrict__ w) {
+  double v[kP], s = 0.0;
+  int at = -1;
+#pragma unroll
+  for (int k = 0; k < kP; ++k) {
+    const double d = t - kNodeX[k];
+    if (d == 0.0) at = k;
+    v[k] = kNodeW[k] / d;
+    s += v[k];
+  }
+  const double r = isfinite(t) ? 1.0 / s : 0.0;
+#pragma unroll
+  for (int k = 0; k < kP; ++k)
+    w[k] = at >= 0 ? (k == at ? 1.0 : 0.0) : r != 0.0 ? v[k] * r : 0.0;
+}
+
+// ---- extents and weights --------------------------------------------------
+
+// Centre and half width of every interval of one axis (level by level); x (n)
+// and the results in LDS.  An interval that holds a value that is not finite
+// is infinitely wide (its centre not a number): no charge is far from it.
+// Called by a whole workgroup; the same result wherever it is computed.
+__device__ __forceinline__ void axis_extents(const float* x, int n, int l, double* m, double* a) {
+  for (int e = threadIdx.x; e < (2 << l) - 1; e += blockDim.x) {
+    const int k = 31 - __clz(e + 1), t = e + 1 - (1 << k);
+    const int i1 = part_begin(n, k, t + 1);
+    float lo = INFINITY, hi = -INFINITY, sum = 0.f;
+#pragma unroll 4
+    for (int i = part_begin(n, k, t); i < i1; ++i) {
+      lo = fminf(lo, x[i]);
+      hi = fmaxf(hi, x[i]);
+      sum += 0.f * x[i];  // not a number for a value that is not finite
+    }
+    const bool fine = sum == 0.f;
+    m[e] = fine ? 0.5 * ((double)lo + (double)hi) : (double)NAN;
+    a[e] = fine ? fmax(0.5 * ((double)hi - (double)lo), 1e-12) : (double)INFINITY;
+  }
+}
+
+// One axis: extents to memory, the weights of its values at every level and
+// the ancestors' weights at the leaf intervals' nodes.
+__device__ void axis_tables(const FarArgs& A, Frame& f, int axis, const float* x,
+                            const double* m, const double* a) {
+  const int n = f.n[axis], l = f.l[axis];
+  double* geo = A.geo + f.geo0 + (long long)axis * kGeoPerAxis * 2;
+  for (int e = threadIdx.x; e < (2 << l) - 1; e += blockDim.x) {
+    geo[2 * e] = m[e];
+    geo[2 * e + 1] = a[e];
+  }
+  for (int r = threadIdx.x; r < (l + 1) * n; r += blockDim.x) {
+    const int k = r / n, i = r - k * n;
+    int t = (int)(((long long)i << k) / n);  // the part that holds value i, or one off
+    while (t > 0 && i < part_begin(n, k, t)) --t;
+    while (i >= part_begin(n, k, t + 1)) ++t;
+    const int e = (1 << k) - 1 + t;
+    lagrange(((double)x[i] - m[e]) / a[e], A.lag + f.lag0[axis] + (long long)r * kP);
+  }
+  const int rows = (1 << l) * l * kP;
+  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
+    const int j = r % kP, k = (r / kP) % l, t = r / (kP * l);
+    const int e = (1 << l) - 1 + t, anc = (1 << k) - 1 + (t >> (l - k));
+    const double X = fma(a[e], kNodeX[j], m[e]);
+    lagrange((X - m[anc]) / a[anc], A.lag + f.tr0[axis] + (long long)r * kP);
+  }
+}
+
+// Whether a charge is far from the cell with centre m and half widths a.
+__device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], const float (&a)[3]) {
+  const float x[3] = {c.x, c.y, c.z};
+  float d2[3], g2[3];
+  bool ok = fabsf(c.w) < 1e30f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const float d = fabsf(x[i] - m[i]);
+    const float gap = fmaxf(d - a[i], 0.0f);
+    ok = ok && d < kMaxCoord && a[i] < kMaxCoord;
+    d2[i] = d * d;
+    g2[i] = gap * gap;
+  }
+  ok = ok && g2[0] + g2[1] + g2[2] >= kMinGap2;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    ok = ok && fmaf(d2[i], kInvS2, (g2[(i + 1) % 3] + g2[(i + 2) % 3]) * kInvS21) >= a[i] * a[i];
+  return ok;
+}
+
+// One wave per 64 charges: the far mask of every cell (far from it, near all
+// its ancestors) and the near mask of every leaf, so that each charge is in
+// exactly one mask of every leaf's path.  A cell whose parent is near none
+// of the wave's charges is skipped.  Padding is in no mask.  The frame's last
+// three workgroups make the tables of one axis each.
+__global__ __launch_bounds__(64) void far_classify_kernel(FarArgs A) {
+  extern __shared__ char dyn[];
+  Frame& f = frame_of_block(&FarFrame::class_blk0, blockIdx.x);
+  const int b = blockIdx.x - f.class_blk0;
+  float* sx = (float*)dyn;                           // the widest axis
+  const int wide = max(f.n[0], max(f.n[1], f.n[2]));
+  double* sm = (double*)(dyn + ((wide * 4 + 15) & ~15));  // 3 x kGeoPerAxis
+  double* sa = sm + 3 * kGeoPerAxis;
+  unsigned long long* far = (unsigned long long*)(sa + 3 * kGeoPerAxis);  // cells
+  unsigned long long* near = far + f.cells;                               // cells
+  const int lane = threadIdx.x;
+  const int only = b < f.nseg ? -1 : b - f.nseg;  // table workgroups: their axis
+  float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (only < 0) c = A.ch[f.ch0 + (long long)b * 64 + lane];
+  for (int i = 0; i < 3; ++i) {
+    if (only >= 0 && i != only) continue;
+    const float* __restrict__ x = A.ax[i] + f.ax0[i];
+    __syncthreads();
+    for (int k = lane; k < f.n[i]; k += 64) sx[k] = x[k];
+    __syncthreads();
+    axis_extents(sx, f.n[i], f.l[i], sm + i * kGeoPerAxis, sa + i * kGeoPerAxis);
+  }
+  __syncthreads();
+  if (only >= 0) {
+    axis_tables(A, f, only, sx, sm + only * kGeoPerAxis, sa + only * kGeoPerAxis);
+    return;
+  }
+  const bool real = !(c.x == kPadCoord && c.y == kPadCoord && c.z == kPadCoord && c.w == 0.f);
+  const unsigned long long all = __ballot(real);
+  int cell0 = 0, parent0 = 0;
+  for (int level = 0; level < f.levels; ++level) {
+    const int cells = cells_at(f, level);
+    for (int k = 0; k < cells; ++k) {
+      int t[3];
+      cell_parts(f, level, k, t);
+      const unsigned long long pm =
+          level ? near[parent0 + ancestor(f, level - 1, level, t)] : all;
+      unsigned long long mf = 0ull;
+      if (pm) {
+        float m[3], a[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const int e = i * kGeoPerAxis + (1 << axis_level(f, i, level)) - 1 + t[i];
+          m[i] = (float)sm[e];
+          a[i] = (float)sa[e];
+        }
+        mf = __ballot(far_from(c, m, a)) & pm;
+      }
+      if (lane == 0) {
+        far[cell0 + k] = mf;
+        near[cell0 + k] = pm & ~mf;
+      }
+    }
+    __syncthreads();
+    parent0 = cell0;
+    cell0 += cells;
+  }
+  const int leaves = cell0 - parent0;
+  unsigned long long* out = A.mask + f.mask0 + b;
+  for (int k = lane; k < f.cells; k += 64) out[(long long)k * f.nseg] = far[k];
+  for (int k = lane; k < leaves; k += 64)
+    out[(long long)(f.cells + k) * f.nseg] = near[parent0 + k];
+}
+
+// ---- charges of a mask list ------------------------------------------------
+
+// Exclusive prefix counts of the list's nseg masks into off (nseg + 1, LDS);
+// returns the total.  Called by the whole workgroup of T threads; tmp (T).
+template <int T>
+__device__ __forceinline__ int list_prefix(const unsigned long long* __restrict__ mask, int nseg,
+                                           int* off, int* tmp) {
+  const int per = (nseg + T - 1) / T;
+  const int s0 = min((int)threadIdx.x * per, nseg), s1 = min(s0 + per, nseg);
+  int n = 0;
+  for (int s = s0; s < s1; ++s) n += __popcll(mask[s]);
+  int run = n;  // inclusive scan inside the wave, then over the waves
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(run, d);
+    if ((int)(threadIdx.x & 63) >= d) run += v;
+  }
+  if ((threadIdx.x & 63) == 63) tmp[threadIdx.x >> 6] = run;
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    if (w < (int)(threadIdx.x >> 6)) before += tmp[w];
+    total += tmp[w];
+  }
+  int o = before + run - n;
+  for (int s = s0; s < s1; ++s) {
+    off[s] = o;
+    o += __popcll(mask[s]);
+  }
+  if (threadIdx.x == 0) off[nseg] = total;
+  __syncthreads();
+  return total;
+}
+
+// Number of the list's r-th charge.
+__device__ __forceinline__ int list_charge(const unsigned long long* __restrict__ mask, int nseg,
+                                           const int* off, int r) {
+  int lo = 0, hi = nseg - 1;  // the last segment with off <= r
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (off[mid] <= r)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  unsigned long long m = mask[lo];
+  int k = r - off[lo], bit = 0;
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {  // the k-th set bit
+    const int n = __popcll(m & ((1ull << w) - 1ull));
+    if (k >= n) {
+      k -= n;
+      bit += w;
+      m >>= w;
+    }
+  }
+  return lo * 64 + bit;
+}
+
+// ---- node sums ---------------------------------------------------------------
+
+// q / r^3 (and q / r) from the FP32 seed of 1 / r and an FP64 correction:
+// with y the seed and e = 1 - r^2 y^2 (|e| ~ 2e-7), 1/r = y (1 + e/2) and
+// 1/r^3 = y^3 (1 + 3e/2) up to e^2 ~ 5e-14.
+template <bool E, bool PHI>
+__device__ __forceinline__ void far_pair(double r2, double q, double& s, double& v) {
+  const double y = (double)__builtin_amdgcn_rsqf((float)r2);
+  const double y2 = y * y;
+  const double e = fma(-r2, y2, 1.0);
+  const double qy = q * y;
+  if constexpr (PHI) v = fma(qy, fma(0.5, e, 1.0), v);
+  if constexpr (E) s = (qy * y2) * fma(1.5, e, 1.0);
+}
+
+// Node workgroups of one frame come level by level, (cell, split, third of the
+// nodes) each; one workgroup per leaf follows, which lists its near charges.
+template <bool E, bool PHI>
+__global__ __launch_bounds__(kNodeThreads, 6) void far_nodes_kernel(FarArgs A) {
+  constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
+  constexpr int kAcc = 3 * C;
+  Frame& f = frame_of_block(&FarFrame::node_blk0, blockIdx.x);
+  __shared__ double4 list[kBatch];  // also the groups' sums: 3 x kAcc x kNodeLanes doubles
+  __shared__ int off[kMaxSegs + 1], tmp[kNodeThreads / 64];
+  static_assert(sizeof(list) >= sizeof(double) * kNodeLanes * kAcc, "one group's sums");
+  const int tid = threadIdx.x;
+  int b = blockIdx.x - f.node_blk0;
+  int level = 0, cell0 = 0;
+  long long part = f.part0;
+  for (; level < f.levels; ++level) {
+    const int cells = cells_at(f, level);
+    const int nb = cells * f.splits[level];
+    if (b < nb * kThirds) break;
+    b -= nb * kThirds;
+    part += (long long)nb * C * kNodes;
+    cell0 += cells;
+  }
+  if (level == f.levels) {  // near list of leaf b
+    const unsigned long long* __restrict__ mask = A.mask + f.mask0 + (long long)(f.cells + b) * f.nseg;
+    const int total = list_prefix<kNodeThreads>(mask, f.nseg, off, tmp);
+    int* out = A.near + f.near0 + (long long)b * (64 * f.nseg + 1);
+    if (tid == 0) out[0] = total;
+    for (int r = tid; r < total; r += kNodeThreads) out[1 + r] = list_charge(mask, f.nseg, off, r);
+    return;
+  }
+  const int third = b % kThirds, slot = b / kThirds;
+  const int splits = f.splits[level];
+  const int cell = slot / splits, split = slot % splits;
+  part += (long long)slot * C * kNodes;
+  int t[3];
+  cell_parts(f, level, cell, t);
+  const double* __restrict__ geo = A.geo + f.geo0;
+  int en[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) en[i] = i * kGeoPerAxis + (1 << axis_level(f, i, level)) - 1 + t[i];
+
+  // this thread's three nodes, one (x, y) line, and its share of the charges
+  const int nl = tid % kNodeLanes, group = tid / kNodeLanes;
+  const int line = third * (kP * kP / kThirds) + nl / 4, z0 = (nl & 3) * 3;
+  const double px = fma(geo[2 * en[0] + 1], kNodeX[line / kP], geo[2 * en[0]]);
+  const double py = fma(geo[2 * en[1] + 1], kNodeX[line % kP], geo[2 * en[1]]);
+  double pz[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) pz[k] = fma(geo[2 * en[2] + 1], kNodeX[z0 + k], geo[2 * en[2]]);
+  double acc[3][C];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[k][c] = 0.0;
+
+  const unsigned long long* __restrict__ mask = A.mask + f.mask0 + (long long)(cell0 + cell) * f.nseg;
+  const float4* __restrict__ ch = A.ch + f.ch0;
+  const int total = list_prefix<kNodeThreads>(mask, f.nseg, off, tmp);
+  const int r0 = (int)((long long)total * split / splits);
+  const int r1 = (int)((long long)total * (split + 1) / splits);
+  for (int base = r0; base < r1; base += kBatch) {
+    const int n = min(kBatch, r1 - base);
+    if (tid < n) {
+      const float4 c = ch[list_charge(mask, f.nseg, off, base + tid)];
+      list[tid] = make_double4(c.x, c.y, c.z, c.w);
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int i = group; i < n; i += kNodeGroups) {
+      const double4 s = list[i];
+      const double dx = px - s.x, dy = py - s.y;
+      const double dxy2 = fma(dy, dy, dx * dx);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double dz = pz[k] - s.z;
+        double w = 0.0;
+        far_pair<E, PHI>(fma(dz, dz, dxy2), s.w, w, acc[k][C - 1]);
+        if constexpr (E) {
+          acc[k][0] = fma(w, dx, acc[k][0]);
+          acc[k][1] = fma(w, dy, acc[k][1]);
+          acc[k][2] = fma(w, dz, acc[k][2]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  // the groups' sums, added in order to group 0's
+  double* sums = (double*)list;
+  for (int g = 1; g < kNodeGroups; ++g) {
+    if (group == g) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int c = 0; c < C; ++c) sums[(k * C + c) * kNodeLanes + nl] = acc[k][c];
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[k][c] += sums[(k * C + c) * kNodeLanes + nl];
+    }
+    __syncthreads();
+  }
+  if (group) return;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      A.part[part + (long long)c * kNodes + line * kP + z0 + k] = acc[k][c];
+}
+
+// ---- the splits' sums --------------------------------------------------------
+
+// Threads per value of a level: the more splits, the more.
+__host__ __device__ inline int red_groups(int splits) {
+  return splits >= 24 ? 8 : splits >= 4 ? 4 : 1;
+}
+
+// Workgroups of a level: none where there is one split (its sums are used as
+// they are).
+__host__ __device__ inline int red_blocks(int cells, int C, int splits) {
+  if (splits == 1) return 0;
+  const int per = kRedThreads / red_groups(splits);
+  return (cells * C * kNodes + per - 1) / per;
+}
+
+template <int C>
+__global__ __launch_bounds__(kRedThreads) void far_reduce_kernel(FarArgs A) {
+  Frame& f = frame_of_block(&FarFrame::red_blk0, blockIdx.x);
+  int b = blockIdx.x - f.red_blk0;
+  long long part = f.part0, val = f.val0;
+  int level = 0, values, groups, per;
+  for (;;) {
+    values = cells_at(f, level) * C * kNodes;
+    groups = red_groups(f.splits[level]);
+    per = kRedThreads / groups;
+    const int nb = red_blocks(cells_at(f, level), C, f.splits[level]);
+    if (b < nb) break;
+    b -= nb;
+    part += (long long)values * f.splits[level];
+    val += values;
+    ++level;
+  }
+  const int splits = f.splits[level];
+  const int g = threadIdx.x / per, v = b * per + threadIdx.x % per;
+  __shared__ double sh[kRedThreads];
+  double s = 0.0;
+  if (v < values) {
+    const int cell = v / (C * kNodes), r = v - cell * C * kNodes;
+    const double* p = A.part + part + (long long)cell * splits * C * kNodes + r;
+#pragma unroll 8
+    for (int i = g; i < splits; i += groups) s += p[(long long)i * C * kNodes];
+  }
+  if (groups > 1) {
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    if (g == 0) {
+      s = 0.0;
+      for (int i = 0; i < groups; ++i) s += sh[i * per + threadIdx.x];
+    }
+  }
+  if (g == 0 && v < values) A.val[val + v] = s;
+}
+
+// ---- points --------------------------------------------------------------------
+
+// 1 / r as the direct kernels' potential has it: +inf at r = 0, not a number
+// at r = inf; ye is the field's, which is 0 there (FP32 rsq).
+__device__ __forceinline__ double near_rsqrt(double r2, double& ye) {
+  const double y = (double)__builtin_amdgcn_rsqf((float)r2);
+  const double e = fma(-r2, fmin(y * y, 1.7976931348623157e308), 1.0);
+  const double v = fma(0.5 * y, e, y);
+  ye = y == 0.0 ? 0.0 : v;
+  return v;
+}
+
+template <bool E, bool PHI, bool SOFT>
+__global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kernel(FarArgs A) {
+  constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
+  constexpr int K = 3;  // points per thread along z
+  constexpr int kPC = kPlanes * C;
+  Frame& f = frame_of_block(&FarFrame::eval_blk0, blockIdx.x);
+  const int b = blockIdx.x - f.eval_blk0;
+  const int leaf = b / f.xblocks, xb = b % f.xblocks;
+  const int bottom = f.levels - 1;
+  int t[3];
+  cell_parts(f, bottom, leaf, t);
+  int lo[3], n[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    lo[i] = part_begin(f.n[i], f.l[i], t[i]);
+    n[i] = part_begin(f.n[i], f.l[i], t[i] + 1) - lo[i];
+  }
+  const int x0 = lo[0] + xb * kPlanes;
+  const int np = min(kPlanes, lo[0] + n[0] - x0);
+  if (np <= 0) return;
+  __shared__ double w1[kPC * kP * kP];
+  __shared__ double w2[kPC * kLeafMax * kP];
+  __shared__ double lz[kLeafMax * kP];
+  // first the contracted planes of a level, then the near charges
+  __shared__ union {
+    double wt[kPC * kP * kP];
+    double4 list[kNearLds];
+  } u;
+  double* const wt = u.wt;
+  const int tid = threadIdx.x;
+  const double* __restrict__ lagy =
+      A.lag + f.lag0[1] + ((long long)f.l[1] * f.n[1] + lo[1]) * kP;
+  const double* __restrict__ lagz =
+      A.lag + f.lag0[2] + ((long long)f.l[2] * f.n[2] + lo[2]) * kP;
+  for (int i = tid; i < n[2] * kP; i += kEvalThreads) lz[i] = lagz[i];
+  for (int i = tid; i < kPC * kP * kP; i += kEvalThreads) w1[i] = 0.0;
+  __syncthreads();
+  // Every level's nodes: x contracted at the planes, y and z carried to the
+  // leaf's nodes, summed in w1.
+  long long val = f.val0, part = f.part0;
+  for (int level = 0; level <= bottom; ++level) {
+    const int ax = axis_level(f, 0, level), ay = axis_level(f, 1, level),
+              az = axis_level(f, 2, level);
+    const double* __restrict__ V = (f.splits[level] == 1 ? A.part + part : A.val + val) +
+                                   (long long)ancestor(f, level, bottom, t) * C * kNodes;
+    val += (long long)cells_at(f, level) * C * kNodes;
+    part += (long long)cells_at(f, level) * f.splits[level] * C * kNodes;
+    const double* __restrict__ lagx = A.lag + f.lag0[0] + ((long long)ax * f.n[0] + x0) * kP;
+    const bool same = ay == f.l[1] && az == f.l[2];
+    double* __restrict__ to = same ? w1 : wt;
+    for (int i = tid; i < C * kP * kP; i += kEvalThreads) {
+      const int comp = i / (kP * kP), r = i % (kP * kP);
+      double s[kPlanes] = {};
+#pragma unroll
+      for (int k = 0; k < kP; ++k) {
+        const double v = V[comp * kNodes + k * kP * kP + r];
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p)
+          s[p] = fma(lagx[min(p, np - 1) * kP + k], v, s[p]);
+      }
+#pragma unroll
+      for (int p = 0; p < kPlanes; ++p) {
+        double* o = to + (p * C + comp) * kP * kP + r;
+        *o = same ? *o + s[p] : s[p];
+      }
+    }
+    __syncthreads();
+    if (same) continue;
+    if (ay != f.l[1]) {  // w2 <- Ty wt
+      const double* __restrict__ T = A.lag + f.tr0[1] + ((long long)t[1] * f.l[1] + ay) * kP * kP;
+      for (int i = tid; i < kPC * kP; i += kEvalThreads) {  // one (plane, comp, z) line
+        const int pc = i / kP, c = i % kP;
+        double v[kP];
+#pragma unroll
+        for (int k = 0; k < kP; ++k) v[k] = wt[pc * kP * kP + k * kP + c];
+        for (int j = 0; j < kP; ++j) {
+          double s = 0.0;
+#pragma unroll
+          for (int k = 0; k < kP; ++k) s = fma(T[j * kP + k], v[k], s);
+          w2[pc * kP * kP + j * kP + c] = s;
+        }
+      }
+    } else {
+      for (int i = tid; i < kPC * kP * kP; i += kEvalThreads) w2[i] = wt[i];
+    }
+    __syncthreads();
+    if (az != f.l[2]) {  // w1 += w2 Tz'
+      const double* __restrict__ T = A.lag + f.tr0[2] + ((long long)t[2] * f.l[2] + az) * kP * kP;
+      for (int i = tid; i < kPC * kP; i += kEvalThreads) {  // one (plane, comp, y) line
+        double v[kP];
+#pragma unroll
+        for (int k = 0; k < kP; ++k) v[k] = w2[i * kP + k];
+        for (int j = 0; j < kP; ++j) {
+          double s = 0.0;
+#pragma unroll
+          for (int k = 0; k < kP; ++k) s = fma(T[j * kP + k], v[k], s);
+          w1[i * kP + j] += s;
+        }
+      }
+    } else {
+      for (int i = tid; i < kPC * kP * kP; i += kEvalThreads) w1[i] += w2[i];
+    }
+    __syncthreads();
+  }
+  // contract y
+  for (int i = tid; i < np * C * n[1] * kP; i += kEvalThreads) {
+    const int c = i % kP, j = (i / kP) % n[1], pc = i / (kP * n[1]);
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kP; ++k) s = fma(lagy[j * kP + k], w1[pc * kP * kP + k * kP + c], s);
+    w2[(pc * kLeafMax + j) * kP + c] = s;
+  }
+  const int* __restrict__ near = A.near + f.near0 + (long long)leaf * (64 * f.nseg + 1);
+  const float4* __restrict__ ch = A.ch + f.ch0;
+  const int total = near[0];
+  __syncthreads();
+  // z, the near charges and the store
+  const float* __restrict__ ax = A.ax[0] + f.ax0[0];
+  const float* __restrict__ ay = A.ax[1] + f.ax0[1];
+  const float* __restrict__ az = A.ax[2] + f.ax0[2];
+  double rclamp;
+  near_rsqrt((double)1e-6f, rclamp);
+  const int chunks = (n[2] + K - 1) / K, items = np * n[1] * chunks;
+  for (int i0 = 0; i0 < items; i0 += kEvalThreads) {  // the same rounds for every thread
+    const int i = min(i0 + tid, items - 1);
+    const bool valid = i0 + tid < items;
+    const int k0 = (i % chunks) * K, j = (i / chunks) % n[1], p = i / (chunks * n[1]);
+    double acc[K][C];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[k][c] = 0.0;
+#pragma unroll
+    for (int a = 0; a < kP; ++a)
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const double v = w2[((p * C + c) * kLeafMax + j) * kP + a];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          acc[k][c] = fma(lz[min(k0 + k, n[2] - 1) * kP + a], v, acc[k][c]);
+      }
+    const double px = ax[x0 + p], py = ay[lo[1] + j];
+    double pz[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) pz[k] = az[lo[2] + min(k0 + k, n[2] - 1)];
+    for (int q0 = 0; q0 < total; q0 += kNearLds) {
+      const int qn = min(kNearLds, total - q0);
+      if (i0 == 0 || total > kNearLds) {  // a short list stays staged
+        __syncthreads();
+        if (tid < qn) {
+          const float4 c = ch[near[1 + q0 + tid]];
+          u.list[tid] = make_double4(c.x, c.y, c.z, c.w);
+        }
+        __syncthreads();
+      }
+      for (int q = 0; q < qn; ++q) {
+        const double4 c = u.list[q];
+        const double dx = px - c.x, dy = py - c.y;
+        const double dxy2 = fma(dy, dy, dx * dx);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const double dz = pz[k] - c.z;
+          double ye;
+          const double y = near_rsqrt(fma(dz, dz, dxy2), ye);
+          if constexpr (PHI) acc[k][C - 1] = fma(c.w, y, acc[k][C - 1]);
+          if constexpr (E) {
+            const double re = SOFT ? fmin(ye, rclamp) : ye;
+            const double w = (c.w * re) * (re * re);
+            acc[k][0] = fma(w, dx, acc[k][0]);
+            acc[k][1] = fma(w, dy, acc[k][1]);
+            acc[k][2] = fma(w, dz, acc[k][2]);
+          }
+        }
+      }
+    }
+    if (!valid) continue;
+    const long long m0 = f.out0 + ((long long)(x0 + p) * f.n[1] + lo[1] + j) * f.n[2] + lo[2] + k0;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (k0 + k < n[2]) {
+        if constexpr (E) {
+          float* e = (float*)A.e + 3 * (m0 + k);
+          e[0] = (float)(kCoulomb * acc[k][0]);
+          e[1] = (float)(kCoulomb * acc[k][1]);
+          e[2] = (float)(kCoulomb * acc[k][2]);
+        }
+        if constexpr (PHI) ((float*)A.phi)[m0 + k] = (float)(kCoulomb * acc[k][C - 1]);
+      }
+  }
+}
+
+int halvings(int n) {
+  int l = 0;
+  while (((n + (1 << l) - 1) >> l) > kLeafMax) ++l;
+  return l;
+}
+
+struct Blocks {
+  long long classify = 0, nodes = 0, reduce = 0, eval = 0;
+  size_t lds = 0;  // of the classification
+};
+
+template <bool E, bool PHI>
+void far_launch(hipStream_t st, const FarArgs& A, const Blocks& n, bool soft) {
+  constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
+  hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(64), n.lds, st, A);
+  hipLaunchKernelGGL((far_nodes_kernel<E, PHI>), dim3((unsigned)n.nodes), dim3(kNodeThreads), 0, st,
+                     A);
+  if (n.reduce)
+    hipLaunchKernelGGL((far_reduce_kernel<C>), dim3((unsigned)n.reduce), dim3(kRedThreads), 0, st,
+                       A);
+  if (soft)
+    hipLaunchKernelGGL((far_eval_kernel<E, PHI, true>), dim3((unsigned)n.eval), dim3(kEvalThreads),
+                       0, st, A);
+  else
+    hipLaunchKernelGGL((far_eval_kernel<E, PHI, false>), dim3((unsigned)n.eval),
+                       dim3(kEvalThreads), 0, st, A);
+}
+
+}  // namespace
+
+bool far_grid_ok(int nx, int ny, int nz, int npad, double min_pairs) {
+  const int n[3] = {nx, ny, nz};
+  for (int i = 0; i < 3; ++i)
+    if (n[i] < kFarMinAxis || n[i] > kMaxAxis) return false;
+  return npad <= 64 * kMaxSegs && (double)nx * ny * nz * npad >= min_pairs;
+}
+
+// Runs the frames in as few groups as the scratch bound allows.
+int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const float* const (&ax)[3],
+                    const float4* ch, bool want_e, bool want_phi, bool soft, void* e, void* phi) {
+  const int C = (want_e ? 3 : 0) + (want_phi ? 1 : 0);
+  constexpr size_t kMaxScratch = (size_t)1 << 30;
+  const int F = (int)grids.size();
+  int done = 0;
+  while (done < F) {
+    std::vector<FarFrame> fr;
+    long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, near = 0;
+    Blocks n;
+    // Node workgroups: two per CU over all frames, shared out by work.  A
+    // level's far charges, over all its cells, are about the charges of the
+    // frame (level 0) or twice that: with kRho, most charges of a level's
+    // near region are far from its children.
+    auto weight = [](int level) { return level ? 2.0 : 1.0; };
+    double work = 0.0;
+    for (int i = done; i < F; ++i) {
+      int deep = 0;
+      for (int k = 0; k < 3; ++k) deep = std::max(deep, halvings(grids[i].n[k]));
+      for (int k = 0; k <= deep; ++k) work += weight(k) * grids[i].npad;
+    }
+    const double quantum = work * kThirds / (2.0 * ctx->num_cus);
+    while (done < F) {
+      const FarGrid& g = grids[done];
+      FarFrame f = {};
+      int wide = 0;
+      for (int i = 0; i < 3; ++i) {
+        f.n[i] = g.n[i];
+        f.l[i] = halvings(g.n[i]);
+        f.ax0[i] = g.ax0[i];
+        f.levels = std::max(f.levels, f.l[i] + 1);
+        wide = std::max(wide, g.n[i]);
+      }
+      f.nseg = g.npad / 64;
+      f.ch0 = g.ch0;
+      f.out0 = g.out0;
+      f.class_blk0 = (int)n.classify;
+      f.node_blk0 = (int)n.nodes;
+      f.red_blk0 = (int)n.reduce;
+      f.eval_blk0 = (int)n.eval;
+      f.part0 = part;
+      f.val0 = val;
+      f.geo0 = geo;
+      f.mask0 = mask;
+      f.near0 = near;
+      long long p = 0, nb = 0, rb = 0, leaves = 0;
+      for (int k = 0; k < f.levels; ++k) {
+        leaves = cells_at(f, k);
+        f.cells += (int)leaves;
+        f.splits[k] = std::max(1, std::min((f.nseg + 1) / 2,
+                                           (int)(weight(k) * g.npad / (leaves * quantum) + 0.5)));
+        nb += leaves * f.splits[k] * kThirds;
+        p += leaves * f.splits[k] * C * kNodes;
+        rb += red_blocks((int)leaves, C, f.splits[k]);
+      }
+      const long long v = (long long)f.cells * C * kNodes;
+      const long long mk = (f.cells + leaves) * f.nseg;
+      const long long nr = leaves * (64LL * f.nseg + 1);
+      if (!fr.empty() &&
+          (size_t)(part + p + val + v + mask + mk) * 8 + (size_t)(near + nr) * 4 > kMaxScratch)
+        break;
+      const int widest = (f.n[0] + (1 << f.l[0]) - 1) >> f.l[0];
+      f.xblocks = (widest + kPlanes - 1) / kPlanes;
+      for (int i = 0; i < 3; ++i) {
+        f.lag0[i] = lag;
+        lag += (long long)(f.l[i] + 1) * f.n[i] * kP;
+        f.tr0[i] = lag;
+        lag += (long long)(1 << f.l[i]) * f.l[i] * kP * kP;
+      }
+      part += p;
+      val += v;
+      mask += mk;
+      near += nr;
+      geo += 3LL * kGeoPerAxis * 2;
+      n.classify += f.nseg + 3;
+      n.nodes += nb + leaves;
+      n.reduce += rb;
+      n.eval += leaves * f.xblocks;
+      n.lds = std::max(n.lds, (size_t)((wide * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
+                                  (size_t)f.cells * 16);
+      fr.push_back(f);
+      ++done;
+    }
+    void* buf = nullptr;
+    int rc = ctx_buf(ctx, kSlotFarGrid, (size_t)(part + val + geo + lag + mask) * 8 + (size_t)near * 4, &buf);
+    if (rc) return rc;
+    FarArgs A = {};
+    A.F = (int)fr.size();
+    A.ch = ch;
+    for (int i = 0; i < 3; ++i) A.ax[i] = ax[i];
+    A.part = (double*)buf;
+    A.val = A.part + part;
+    A.geo = A.val + val;
+    A.lag = A.geo + geo;
+    A.mask = (unsigned long long*)(A.lag + lag);
+    A.near = (int*)(A.mask + mask);
+    A.e = e;
+    A.phi = phi;
+    if (A.F == 1) {
+      A.one = fr[0];
+    } else {
+      void* tab = nullptr;
+      if ((rc = ctx_buf(ctx, kSlotFarTables, fr.size() * sizeof(FarFrame), &tab))) return rc;
+      if ((rc = upload_table(ctx, kTabFarFrames, tab, fr.data(), fr.size() * sizeof(FarFrame))))
+        return rc;
+      A.frames = (const FarFrame*)tab;
+    }
+    if (want_e && want_phi)
+      far_launch<true, true>(ctx->stream, A, n, soft);
+    else if (want_e)
+      far_launch<true, false>(ctx->stream, A, n, soft);
+    else
+      far_launch<false, true>(ctx->stream, A, n, soft);
+    CPET_HIP_TRY(hipGetLastError());
+  }
+  return CPET_OK;
+}
+
+}  // namespace cpet
