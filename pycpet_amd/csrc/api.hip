@@ -189,6 +189,27 @@ int ctx_buf(cpet_ctx* ctx, int slot, size_t bytes, void** out) {
   return CPET_OK;
 }
 
+void* ctx_buf_try(cpet_ctx* ctx, int slot, size_t bytes) {
+  void* p = nullptr;
+  if (ctx->arena) {
+    const size_t off = (ctx->arena_used + 255) & ~(size_t)255;
+    if (off > ctx->arena_bytes || bytes > ctx->arena_bytes - off) return nullptr;
+  } else if (ctx->bufs[slot].bytes < bytes) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  const std::string before = g_err;
+  if (ctx_buf(ctx, slot, bytes, &p)) {
+    (void)hipGetLastError();  // an allocation that failed
+    set_error("%s", before.c_str());
+    return nullptr;
+  }
+  return p;
+}
+
 int upload_table(cpet_ctx* ctx, int key, void* dst, const void* src, size_t bytes) {
   auto& t = ctx->tables[key];
   const char* d = (const char*)dst;

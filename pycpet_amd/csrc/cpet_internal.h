@@ -145,12 +145,17 @@ enum Slot : int {
   kSlotFar,          // streamlines: far-field charge records + per-frame flags
   kSlotFarGrid,      // interpolating grid path: node sums, weights, near lists
   kSlotFarTables,    // its frames (written by upload_table only)
+  kSlotChunks,       // streamlines: sources in the order of the chunk-lane form
   kSlotCount
 };
 
 // Returns a device buffer of at least `bytes` for `slot`, growing it if needed
 // (or, for a context with an arena, a region of the arena).
 int ctx_buf(cpet_ctx* ctx, int slot, size_t bytes, void** out);
+// The same for a buffer that the call can do without: null where it would not
+// fit the arena, or would have to be allocated while the stream is being
+// captured, or memory has run out.
+void* ctx_buf_try(cpet_ctx* ctx, int slot, size_t bytes);
 // Forgets the arena regions of the previous call.
 void arena_reset(cpet_ctx* ctx);
 // cpet_topo after argument validation, with the context locked and active.

@@ -219,6 +219,8 @@ struct PropArgs {
   double4* res;     // (L) final point, steps and stop kind (ResultRec)
   unsigned int* counter;
   const int* far_unsafe;   // null (no far-field form), or 0: every charge is far
+  const float4* chunks;    // chunk groups (chunk_pack_kernel), or null
+  int slots;               // slots a workgroup uses, of 64
 };
 
 // Streams source records [r0, r1) (float4; r0 and r1 multiples of four) to
@@ -328,28 +330,117 @@ __device__ __forceinline__ void wave_records(int rec0, int nrec, int wave, int S
   r1 = rec0 + (int)((wave + 1) * n / S) * gran;
 }
 
+// ---- chunk-lane form of the slice sums ----------------------------------
+//
+// A streamline's steps follow one another, so a workgroup whose slots are
+// mostly done (or that never had 64 streamlines) is bound by the time of one
+// evaluation: in the slice form, where a lane is a slot, that is the whole
+// slice whatever the number of slots in use.  The sums are FP32 over chunks
+// of 64 sources and FP64 over a slice's chunks, so the chunks are
+// independent: in this form the 64 lanes of a wave take four slots x the
+// j-th chunk of all 16 slices, and the waves share the (slot quad, j) tasks.
+// Idle slots cost nothing, every lane works, and the chunk sums, their order
+// inside a slice and the order of the slices are those of the slice form: the
+// results are the same bit for bit.
+//
+// Lane 4b + i of a wave serves slot i of the quad and slice b.  Each lane
+// loads one source of its slice's chunk (lane 4b + i source i of four), and
+// v_mfma_f32_4x4x1 (16 blocks of a 4 x 1 by 1 x 4 product) hands all four to
+// the block's four lanes: x_source * -1 + p, one product and one addition of
+// exact operands, is the subtraction p - x_source, and w * 1 + 0 is w.  That
+// leaves 10 of a pair's 13 vector operations; with the loads, the matrix
+// instructions and the barriers a pair and wave takes 52 cycles against the
+// slice form's 45.  The broadcast as a DPP operand of the 13 operations
+// takes 61: such an operand costs a second pass.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kChunk = kTile;           // sources of an FP32 sum
+constexpr int kChunkQuads = kChunk / 4;
+constexpr int kSplitSlices = 16;        // slices of the 16-wave kernel
+constexpr int kChunkSums = 16 * 3 * 512;  // FP32 chunk sums in LDS at once (96 KB)
+// Pairs per lane that the form has to save: its extra barrier and LDS trips
+// take about the time of two chunks of one wave.
+constexpr int kSplitGain = 128;
+
+template <int K>
+__device__ __forceinline__ void quad_displace(const float4& c, const f32x4 (&p)[3],
+                                              f32x4 (&d)[K]) {
+  d[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(c.x, -1.f, p[0], 0, 0, 0);
+  d[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(c.y, -1.f, p[1], 0, 0, 0);
+  d[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(c.z, -1.f, p[2], 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 quad_spread(float w) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(w, 1.f, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+}
+
+// Number of chunk groups (the j-th chunks of all slices) that a frame of npad
+// padded sources has at most, and of the frames before frame f of a batch
+// (their source offset c0, a multiple of kTile): an upper bound that needs no
+// table.
+__host__ __device__ inline int chunk_groups(int npad) {
+  return (npad + kSplitSlices * kChunk - 1) / (kSplitSlices * kChunk);
+}
+__host__ __device__ inline int chunk_group0(int c0, int f) {
+  return c0 / (kSplitSlices * kChunk) + f;
+}
+
+// Sources of the longest of the kSplitSlices slices of nrec records, rps per
+// source (both forms cut at whole groups of four records).
+__device__ __forceinline__ int longest_slice(int nrec, int rps) {
+  return (nrec / 4 + kSplitSlices - 1) / kSplitSlices * 4 / rps;
+}
+
 // Sources of the field a streamline follows.  A policy gives the FP32
 // slice sum of the propagate kernel and the FP64 field of the epilogue.
 //
+// The 13 operations of a pair are kept together, in the order in which one
+// needs the other (a scheduling barrier after each pair).  The scheduler's own
+// order, which starts the next pairs during a pair's rsq, looks better and is
+// slower: 53.8 against 45.0 cycles a pair and wave in a loop of the pairs alone
+// (four waves per SIMD), and hand-made mixtures of two or four pairs take 46
+// to 51.  Four waves per SIMD fill a wave's waits anyway.  The one-wave walk of
+// a few sources goes without (2 % slower with it).
+template <bool ORDER>
+__device__ __forceinline__ void pair_order() {
+  if constexpr (ORDER) __builtin_amdgcn_sched_barrier(0);
+}
+
 // Charges: one float4 (x, y, z, q) per source (math_module.c:296-333).
 struct ChargeSrc {
   static constexpr int kRecPerSrc = 1;
   static constexpr int kComp = 3;  // the slice sums are the field components
   // Unsoftened field of charge records [r0, r1) at one point (the k factor
   // is applied by the caller).
+  // The FP32 term of one charge at displacement d, added into f.
+  template <bool ORDER = true>
+  __device__ static void pair(float dx, float dy, float dz, float q, float (&f)[3]) {
+    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    const float ri = __builtin_amdgcn_rsqf(r2);
+    const float s = (q * ri) * (ri * ri);
+    f[0] = fmaf(s, dx, f[0]);
+    f[1] = fmaf(s, dy, f[1]);
+    f[2] = fmaf(s, dz, f[2]);
+    pair_order<ORDER>();
+  }
   // The FP32 terms of one group of four charge records, added into f.
+  template <bool ORDER = true>
   __device__ static void group(float px, float py, float pz, const float4 (&c)[4],
                                float (&f)[3]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const float dx = px - c[u].x, dy = py - c[u].y, dz = pz - c[u].z;
-      const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-      const float ri = __builtin_amdgcn_rsqf(r2);
-      const float s = (c[u].w * ri) * (ri * ri);
-      f[0] = fmaf(s, dx, f[0]);
-      f[1] = fmaf(s, dy, f[1]);
-      f[2] = fmaf(s, dz, f[2]);
-    }
+    for (int u = 0; u < 4; ++u)
+      pair<ORDER>(px - c[u].x, py - c[u].y, pz - c[u].z, c[u].w, f);
+  }
+  // Displacements and charges of four charges, charge i of them in lane
+  // 4b + i of each block of four lanes (see quad_displace), and their terms.
+  static constexpr int kSpread = 4;
+  __device__ static void spread(const float4 (&c)[1], const f32x4 (&p)[3], f32x4 (&d)[4]) {
+    quad_displace(c[0], p, d);
+    d[3] = quad_spread(c[0].w);
+  }
+  __device__ static void quad(const f32x4 (&d)[4], float (&f)[3]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pair(d[0][u], d[1][u], d[2][u], d[3][u], f);
   }
   __device__ static void slice(float px, float py, float pz, const float4* __restrict__ ch,
                                int r0, int r1, double (&e)[3]) {
@@ -396,22 +487,42 @@ struct DipoleSrc {
   __device__ static float coef(float mx, float my, float mz, float dx, float dy, float dz) {
     return PHYS ? 3.f * fmaf(mz, dz, fmaf(my, dy, mx * dx)) : fmaf(3.f * mx, dx, fmaf(my, dy, mz * dz));
   }
+  // The FP32 term of one dipole at displacement d, added into f.
+  template <bool ORDER = true>
+  __device__ static void pair(float dx, float dy, float dz, float mx, float my, float mz,
+                              float (&f)[3]) {
+    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    const float ri = __builtin_amdgcn_rsqf(r2);
+    const float ri2 = ri * ri;
+    const float ri5 = (ri2 * ri2) * ri;
+    const float cc = coef(mx, my, mz, dx, dy, dz);
+    f[0] = fmaf(ri5, fmaf(cc, dx, -mx * r2), f[0]);
+    f[1] = fmaf(ri5, fmaf(cc, dy, -my * r2), f[1]);
+    f[2] = fmaf(ri5, fmaf(cc, dz, -mz * r2), f[2]);
+    pair_order<ORDER>();
+  }
   // The FP32 terms of one group of four records (two dipoles), added into f.
+  template <bool ORDER = true>
   __device__ static void group(float px, float py, float pz, const float4 (&c)[4],
                                float (&f)[3]) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const float4 X = c[2 * u], M = c[2 * u + 1];
-      const float dx = px - X.x, dy = py - X.y, dz = pz - X.z;
-      const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-      const float ri = __builtin_amdgcn_rsqf(r2);
-      const float ri2 = ri * ri;
-      const float ri5 = (ri2 * ri2) * ri;
-      const float cc = coef(M.x, M.y, M.z, dx, dy, dz);
-      f[0] = fmaf(ri5, fmaf(cc, dx, -M.x * r2), f[0]);
-      f[1] = fmaf(ri5, fmaf(cc, dy, -M.y * r2), f[1]);
-      f[2] = fmaf(ri5, fmaf(cc, dz, -M.z * r2), f[2]);
+      pair<ORDER>(px - X.x, py - X.y, pz - X.z, M.x, M.y, M.z, f);
     }
+  }
+  // As ChargeSrc::spread and quad, of four dipoles.
+  static constexpr int kSpread = 6;
+  __device__ static void spread(const float4 (&c)[2], const f32x4 (&p)[3], f32x4 (&d)[6]) {
+    quad_displace(c[0], p, d);
+    d[3] = quad_spread(c[1].x);
+    d[4] = quad_spread(c[1].y);
+    d[5] = quad_spread(c[1].z);
+  }
+  __device__ static void quad(const f32x4 (&d)[6], float (&f)[3]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      pair(d[0][u], d[1][u], d[2][u], d[3][u], d[4][u], d[5][u], f);
   }
   __device__ static void slice(float px, float py, float pz, const float4* __restrict__ ch,
                                int r0, int r1, double (&e)[3]) {
@@ -620,6 +731,96 @@ __global__ __launch_bounds__(256) void far_pack_kernel(int total, const float4* 
   if (!(reach <= (double)kFarRatio * dist)) unsafe[fr] = 1;
 }
 
+// The sources in the order of the chunk-lane form: group j, quad t, record k
+// of a source, lane 4b + i: source 64 j + 4 t + i of slice b, or padding past
+// the slice's end.  One block per quarter of a group; chg_off (F+1) are the
+// padded source offsets of a batch, null for one frame of npad sources.
+template <int RPS>
+__global__ __launch_bounds__(256) void chunk_pack_kernel(const float4* __restrict__ ch, int F,
+                                                         const int32_t* __restrict__ chg_off,
+                                                         int npad, float4* __restrict__ out) {
+  const int group = blockIdx.x >> 2;
+  const int lane = threadIdx.x & 63, t = (blockIdx.x & 3) * 4 + (threadIdx.x >> 6);
+  int fr = 0, c0 = 0, n = npad;
+  if (chg_off) {
+    int lo = 0, hi = F - 1;  // the last frame whose first group is <= group
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (chunk_group0(chg_off[mid], mid) <= group)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    fr = lo;
+    c0 = chg_off[fr];
+    n = chg_off[fr + 1] - c0;
+  }
+  const int j = group - chunk_group0(c0, fr);
+  if (j >= chunk_groups(n)) return;  // a gap between frames
+  const int nrec = used_records(ch, c0 * RPS, n * RPS, RPS, lane);
+  int r0, r1;
+  wave_records(c0 * RPS, nrec, lane >> 2, kSplitSlices, r0, r1);
+  const int r = r0 + (j * kChunk + 4 * t + (lane & 3)) * RPS;
+  float4 rec[RPS];
+#pragma unroll
+  for (int k = 0; k < RPS; ++k)
+    rec[k] = k ? make_float4(0.f, 0.f, 0.f, 0.f)
+               : make_float4(kPadCoord, kPadCoord, kPadCoord, 0.f);
+  if (r < r1)
+#pragma unroll
+    for (int k = 0; k < RPS; ++k) rec[k] = ch[r + k];
+  float4* o = out + ((size_t)(group * kChunkQuads + t) * RPS) * 64 + lane;
+#pragma unroll
+  for (int k = 0; k < RPS; ++k) o[k * 64] = rec[k];
+}
+
+// The FP32 sums of one chunk per lane (chunk_pack_kernel's group `rec`, its
+// first `quads` quads) at the lane's point.  The sources of the next four
+// quads (two, of two-record sources) are loaded during the arithmetic of the
+// current ones, into two buffers in turn, and the next quad's displacements
+// run on the matrix unit during the current quad's pairs.
+template <class Src>
+__device__ __forceinline__ void chunk_sums(const float4* __restrict__ rec, int quads, float px,
+                                           float py, float pz, int lane, float (&f)[3]) {
+  constexpr int R = Src::kRecPerSrc, H = 4 / R, K = Src::kSpread;
+  static_assert(H % 2 == 0, "the quads alternate between two buffers");
+  const f32x4 p[3] = {{px, px, px, px}, {py, py, py, py}, {pz, pz, pz, pz}};
+  float4 c[2 * H][R];
+  f32x4 d[2][K];
+  auto load = [&](int half, int t) __attribute__((always_inline)) {
+    const float4* __restrict__ at = rec + t * R * 64 + lane;
+#pragma unroll
+    for (int u = 0; u < H; ++u)
+#pragma unroll
+      for (int k = 0; k < R; ++k) c[half * H + u][k] = at[(u * R + k) * 64];
+  };
+  // quad u of the 2 H in c, after starting on the one behind it
+  auto step = [&](int u) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    Src::spread(c[(u + 1) % (2 * H)], p, d[(u + 1) & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    Src::quad(d[u & 1], f);
+  };
+  load(0, 0);
+  Src::spread(c[0], p, d[0]);
+  int t = 0;
+#pragma unroll 1
+  for (; t + 2 * H <= quads; t += 2 * H) {
+    load(1, t + H);
+#pragma unroll
+    for (int u = 0; u < H; ++u) step(u);
+    load(0, min(t + 2 * H, kChunkQuads - H));
+#pragma unroll
+    for (int u = H; u < 2 * H; ++u) step(u);
+  }
+  if (t < quads) {  // t + 2 H <= kChunkQuads: a multiple of 2 H below it
+    load(1, t + H);
+#pragma unroll
+    for (int u = 0; u < 2 * H - 1; ++u)
+      if (t + u < quads) step(u);
+  }
+}
+
 enum SlotState : int { kActive = 0, kNeed = 1, kDone = 2 };
 
 // Result record of one streamline, written once when it stops: the final
@@ -645,6 +846,8 @@ struct FrameView {
   unsigned int* counter;   // next queue position
   int r0, r1;              // this wave's source records (float4)
   int vrec0, vnrec, vgran;  // the frame's used records and split granule (S == 1 walk)
+  const float4* chunks;    // its chunk groups (16-wave workgroups), or null
+  int slice;               // sources of its longest slice
 };
 
 // A one-wave workgroup (S == 1) walks the kVirtWaves slices of the
@@ -670,7 +873,7 @@ constexpr int kVirtMinStarts = 50000;  // at least this many starts
 // one partial buffer suffices (S < 4 alternates two).  A finished slot asks
 // the queue for the next streamline (one idle iteration).  first_q >= 0
 // gives the slot an initial queue position, first_q < 0 starts it empty.
-// part holds kPartBufs(S) * S * 4 * 64 doubles, esum 4 * 64.
+// part holds kPartBufs(S) * S * NC * 64 doubles, esum NC * 64.
 // The one-wave walk, general form: the kVirtWaves slices in order, each
 // summed by the policy's slice exactly as its wave of the kVirtWaves-wave
 // split would, added into fc (which starts at 0) in that order.  An empty
@@ -717,7 +920,7 @@ __device__ __forceinline__ void walk_groups(float px, float py, float pz,
   for (int u = 0; u < 4; ++u) a[u] = ch[nx + u];
   auto one = [&](const float4 (&c)[4]) __attribute__((always_inline)) {
     float g[3] = {0.f, 0.f, 0.f};
-    Src::group(px, py, pz, c, g);
+    Src::template group<false>(px, py, pz, c, g);
 #pragma unroll
     for (int k = 0; k < 3; ++k) fc[k] += (double)g[k];
   };
@@ -743,10 +946,66 @@ __device__ __forceinline__ void walk_groups(float px, float py, float pz,
 
 __host__ __device__ constexpr int kPartBufs(int S) { return S >= 4 ? 1 : 2; }
 
+// Whether the kernel of S waves and these sources has the chunk-lane form.
+template <int S, class Src>
+struct HasChunks {
+  static constexpr bool value = S == kSplitSlices && HasGroup<Src>::value;
+};
+
+// The chunk-lane form of one evaluation of the workgroup's active slots: the
+// calling wave's slice sums go into fc.  Called by all waves with the same
+// slot state; e32 is the lane's slot's point.  cs (kChunkSums) is free.
+template <class Src>
+__device__ __forceinline__ void split_slices(const FrameView& f, unsigned long long act, float ex,
+                                             float ey, float ez, float* cs, int lane, int wave,
+                                             double (&fc)[3]) {
+  const int k = __popcll(act), tiles = (k + 3) >> 2, row = 4 * tiles;
+  const bool active = (act >> lane) & 1;
+  const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(act >> 32),
+                                             __builtin_amdgcn_mbcnt_lo((unsigned)act, 0u));
+  // lane r holds the slot of rank r: the active ones first
+  const int slot_of = __builtin_amdgcn_ds_permute(4 * (active ? rank : k + lane - rank), lane);
+  const int groups = (f.slice + kChunk - 1) / kChunk;
+  const int per = min(groups, kChunkSums / (3 * kSplitSlices) / row);
+  for (int g0 = 0; g0 < groups; g0 += per) {
+    const int ng = min(per, groups - g0);
+    if (g0) __syncthreads();  // the previous groups' sums have been read
+    int j = 0, tile = wave;   // task `wave` of ng x tiles, then every 16th
+    while (tile >= tiles && j < ng) {
+      tile -= tiles;
+      ++j;
+    }
+    while (j < ng) {
+      const int r = 4 * tile + (lane & 3);
+      const int s = __shfl(slot_of, r);
+      const float px = __shfl(ex, s), py = __shfl(ey, s), pz = __shfl(ez, s);
+      const int left = f.slice - (g0 + j) * kChunk;  // sources of the longest chunk
+      float c[3] = {0.f, 0.f, 0.f};
+      chunk_sums<Src>(f.chunks + (size_t)(g0 + j) * kChunkQuads * Src::kRecPerSrc * 64,
+                      min(kChunkQuads, (left + 3) >> 2), px, py, pz, lane, c);
+      float* o = cs + ((j * kSplitSlices + (lane >> 2)) * 3) * row + r;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) o[i * row] = c[i];
+      tile += kSplitSlices;
+      while (tile >= tiles && j < ng) {
+        tile -= tiles;
+        ++j;
+      }
+    }
+    __syncthreads();
+    // a chunk past a slice's end holds +0, which changes no sum
+    if (active)
+      for (int j = 0; j < ng; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          fc[i] += (double)cs[((j * kSplitSlices + wave) * 3 + i) * row + rank];
+  }
+}
+
 template <int S, class Src>
 __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const FrameView& f,
                                           int first_q, double* part, double* esum,
-                                          int (*nsid)[64], int lane, int wave) {
+                                          int (*nsid)[64], float* cs, int lane, int wave) {
   constexpr bool rk4 = IsRk4<Src>::value;
   constexpr int NC = Src::kComp;
   constexpr int NB = kPartBufs(S);
@@ -785,7 +1044,7 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
   if (first_q >= 0)
     load(first_q);
   else
-    st = kNeed;
+    st = lane < -first_q ? kNeed : kDone;
   int par = 0;
   while (__ballot(st != kDone) != 0ull) {
     double fc[NC];
@@ -794,7 +1053,16 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
     // the evaluation point as the FP32 slice sees it
     const float ex32 = (float)(rk4 ? qx : px), ey32 = (float)(rk4 ? qy : py),
                 ez32 = (float)(rk4 ? qz : pz);
-    if (st == kActive) {
+    const unsigned long long act = __ballot(st == kActive);
+    // the slice form takes 16 x slice pairs' time a wave, the chunk-lane form
+    // that of its slot quads (of 16)
+    bool split = false;
+    if constexpr (HasChunks<S, Src>::value) {
+      const int tiles = (__popcll(act) + 3) >> 2;
+      split = f.chunks && tiles > 0 && (15 - tiles) * f.slice >= kSplitGain;
+      if (split) split_slices<Src>(f, act, ex32, ey32, ez32, cs, lane, wave, fc);
+    }
+    if (st == kActive && !split) {
       if constexpr (S == 1 && HasGroup<Src>::value) {
         if (f.vnrec <= kVirtWaves * 4) {
           walk_groups<Src>(ex32, ey32, ez32, ch, f.vrec0, f.vnrec, fc);
@@ -910,15 +1178,26 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
   }
 }
 
+// A slot's first place in the queue: the places go round the workgroups, so
+// that each has a like share of the long streamlines.  A slot that is not used
+// gets one past the end.
+__device__ __forceinline__ int first_place(const PropArgs& a, int lane) {
+  return lane < a.slots ? lane * (int)gridDim.x + (int)blockIdx.x : a.L;
+}
+
 // Single frame.  The charge pointer is a separate __restrict__ parameter so
 // the compiler may read charges through the scalar cache despite the
 // kernel's stores.
+//
+// The 16-wave workgroup is alone on its CU (its LDS, and one per CU is what
+// is launched), four waves per SIMD.
 template <int S, class Src>
-__global__ __launch_bounds__(64 * S, 8) void topo_propagate_kernel(
+__global__ __launch_bounds__(64 * S, S >= 16 ? 4 : 8) void topo_propagate_kernel(
     const float4* __restrict__ ch, PropArgs a) {
-  __shared__ double part[kPartBufs(S) * S * 4 * 64];
-  __shared__ double esum[4 * 64];
+  __shared__ double part[kPartBufs(S) * S * Src::kComp * 64];
+  __shared__ double esum[Src::kComp * 64];
   __shared__ int nsid[2][64];
+  __shared__ float cs[HasChunks<S, Src>::value ? kChunkSums : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   FrameView f;
@@ -940,7 +1219,9 @@ __global__ __launch_bounds__(64 * S, 8) void topo_propagate_kernel(
   f.vrec0 = 0;
   f.vnrec = nrec;
   f.vgran = 4;
-  run_slots<S, Src>(ch, f, blockIdx.x * 64 + lane, part, esum, nsid, lane, wave);
+  f.chunks = a.chunks;
+  f.slice = longest_slice(nrec, Src::kRecPerSrc);
+  run_slots<S, Src>(ch, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
 }
 
 // The far-field form (ChargeSrcFar) of the single-frame kernel, launched
@@ -951,9 +1232,10 @@ __global__ __launch_bounds__(64 * S, 8) void topo_propagate_kernel(
 template <int S>
 __global__ __launch_bounds__(64 * S, 4) void topo_far_kernel(const float4* __restrict__ far,
                                                            PropArgs a) {
-  __shared__ double part[kPartBufs(S) * S * 4 * 64];
-  __shared__ double esum[4 * 64];
+  __shared__ double part[kPartBufs(S) * S * ChargeSrcFar::kComp * 64];
+  __shared__ double esum[ChargeSrcFar::kComp * 64];
   __shared__ int nsid[2][64];
+  __shared__ float cs[HasChunks<S, ChargeSrcFar>::value ? kChunkSums : 1];
   if (__builtin_amdgcn_readfirstlane(*a.far_unsafe) != 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -974,7 +1256,9 @@ __global__ __launch_bounds__(64 * S, 4) void topo_far_kernel(const float4* __res
   f.vrec0 = 0;
   f.vnrec = nrec;
   f.vgran = gran;
-  run_slots<S, ChargeSrcFar>(far, f, blockIdx.x * 64 + lane, part, esum, nsid, lane, wave);
+  f.chunks = nullptr;
+  f.slice = 0;
+  run_slots<S, ChargeSrcFar>(far, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
 }
 
 // Many frames in one persistent launch.  Workgroups claim assignments
@@ -997,6 +1281,8 @@ struct BatchTopoArgs {
   int n_assign;
   unsigned int* assign_counter;  // [0]: direct-form kernel, [1]: far-form kernel
   const int* far_unsafe;      // (F) 0: frame f's charges are far from its walk region, or null
+  const float4* chunks;       // chunk groups of all frames (chunk_pack_kernel), or null
+  int slots;                  // slots a workgroup uses, of 64
 };
 
 // The batch body for one form: FAR = 0 runs the frames that use the direct
@@ -1007,9 +1293,11 @@ struct BatchTopoArgs {
 // frames, so every frame runs in exactly one of them.
 template <int S, bool FAR>
 __device__ __forceinline__ void batch_body(const float4* __restrict__ src, BatchTopoArgs a) {
-  __shared__ double part[kPartBufs(S) * S * 4 * 64];
-  __shared__ double esum[4 * 64];
+  using Src = typename std::conditional<FAR, ChargeSrcFar, ChargeSrc>::type;
+  __shared__ double part[kPartBufs(S) * S * Src::kComp * 64];
+  __shared__ double esum[Src::kComp * 64];
   __shared__ int nsid[2][64];
+  __shared__ float cs[HasChunks<S, Src>::value ? kChunkSums : 1];
   __shared__ int cur;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1045,20 +1333,24 @@ __device__ __forceinline__ void batch_body(const float4* __restrict__ src, Batch
       f.vrec0 = rps * c0;
       f.vnrec = nrec;
       f.vgran = gran;
-      run_slots<S, ChargeSrcFar>(src, f, -1, part, esum, nsid, lane, wave);
+      f.chunks = nullptr;
+      f.slice = 0;
+      run_slots<S, ChargeSrcFar>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
     } else {
       const int nrec = __builtin_amdgcn_readfirstlane(used_records(src, c0, nc, 1, lane));
       wave_records(c0, nrec, wave, S, f.r0, f.r1);
       f.vrec0 = c0;
       f.vnrec = nrec;
       f.vgran = 4;
-      run_slots<S, ChargeSrc>(src, f, -1, part, esum, nsid, lane, wave);
+      f.chunks = a.chunks ? a.chunks + (size_t)chunk_group0(c0, fr) * kChunkQuads * 64 : nullptr;
+      f.slice = longest_slice(nrec, 1);
+      run_slots<S, ChargeSrc>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
     }
   }
 }
 
 template <int S>
-__global__ __launch_bounds__(64 * S, 8) void topo_batch_kernel(const float4* __restrict__ ch,
+__global__ __launch_bounds__(64 * S, S >= 16 ? 4 : 8) void topo_batch_kernel(const float4* __restrict__ ch,
                                                             BatchTopoArgs a) {
   batch_body<S, false>(ch, a);
 }
@@ -1417,6 +1709,27 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
     d_far_unsafe = flag;
   }
 
+  // chunk groups of the 16-wave workgroups; without them (no room in a fixed
+  // arena, or none yet while the stream is being captured) the kernel keeps
+  // to the slice form, with the same results
+  const bool f64 = src == kSrcChargeF64 || src == kSrcChargeF64Rk4;
+  const int rps = src == kSrcDipoleRef || src == kSrcDipolePhys ? 2 : 1;
+  float4* d_chunks = nullptr;
+  if (S == kSplitSlices && !f64) {
+    const int groups = chunk_groups(npad);
+    d_chunks = (float4*)ctx_buf_try(ctx, kSlotChunks,
+                                    (size_t)groups * kChunkQuads * 64 * rps * sizeof(float4));
+    if (d_chunks) {
+      if (rps == 1)
+        hipLaunchKernelGGL(chunk_pack_kernel<1>, dim3(4 * groups), dim3(256), 0, st, ch, 1,
+                           (const int32_t*)nullptr, npad, d_chunks);
+      else
+        hipLaunchKernelGGL(chunk_pack_kernel<2>, dim3(4 * groups), dim3(256), 0, st, ch, 1,
+                           (const int32_t*)nullptr, npad, d_chunks);
+      CPET_HIP_TRY(hipGetLastError());
+    }
+  }
+
   // 1. longest-first order
   if ((rc = prof_mark(ctx, 0))) return rc;
   hipLaunchKernelGGL(fill_u32_kernel, dim3((kNumBuckets + 255) / 256), dim3(256), 0, st,
@@ -1430,15 +1743,30 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
 
   // 2. propagate
   int G = ctx->tune[2][1];
-  const int gmax = (L + 63) / 64;
+  // with the chunk-lane form a workgroup need not have 64 streamlines: every
+  // CU gets a share
+  const int gmax = d_chunks ? L : (L + 63) / 64;
   // One 16-wave workgroup per CU: the fewest slots that keep every SIMD fed
   // (4 waves each, with the charge loads prefetched), so the tail of long
   // streamlines still running after the queue drains is shortest.
   if (G <= 0)
     G = std::min(gmax, std::max(1, ctx->num_cus * (S >= 16 ? 1 : S == 1 ? 24 : 2)));
   G = std::min(G, gmax);
+  // Where all streamlines would be in slots at once, a workgroup's share of
+  // the steps is settled before it starts, and the largest share is 40 % over
+  // the mean (42 streamlines of a 10,648-streamline frame).  A third of the
+  // slots then leaves two thirds of the streamlines in the queue, for the
+  // workgroups that are done early: 13.0 -> 10.0 ms for that frame of 10,000
+  // charges.  As many slots as give each wave a task (a slot quad and chunk
+  // group) are used in any case: 16 slots of a 300-charge frame took 3.1 ms
+  // against 1.75.
+  int slots = 64;
+  if (d_chunks && L <= 64LL * G) {
+    const int want = std::max((L + 3 * G - 1) / (3 * G), 64 / chunk_groups(npad));
+    slots = std::max(4, std::min(64, (want + 3) / 4 * 4));
+  }
   hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(256), 0, st, d_counter, 1LL,
-                     (unsigned int)(G * 64));
+                     (unsigned int)(G * slots));
   if ((rc = prof_mark(ctx, 1))) return rc;
   PropArgs pa;
   pa.npad = npad;
@@ -1453,6 +1781,8 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
   pa.res = d_res;
   pa.counter = d_counter;
   pa.far_unsafe = d_far_unsafe;
+  pa.chunks = d_chunks;
+  pa.slots = slots;
   if (S != 1 && S != 2 && S != 4 && S != 8 && S != 16) {
     set_error("unsupported waves per workgroup %d (1,2,4,8,16)", S);
     return CPET_ERR_ARG;
@@ -1577,13 +1907,37 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   const int G0 = ctx->tune[3][1] > 0 ? ctx->tune[3][1]
                : S == 1            ? ctx->num_cus * 24
                                    : ctx->num_cus * (S >= 16 ? 1 : 2);
+  // chunk groups of every frame (see topo_run)
+  float4* d_chunks = nullptr;
+  if (S == kSplitSlices) {
+    const int groups = chunk_group0(chg_off[F], F);
+    d_chunks = (float4*)ctx_buf_try(ctx, kSlotChunks,
+                                    (size_t)groups * kChunkQuads * 64 * sizeof(float4));
+    if (d_chunks) {
+      hipLaunchKernelGGL(chunk_pack_kernel<1>, dim3(4 * groups), dim3(256), 0, st, ch, F,
+                         d_chg_off, 0, d_chunks);
+      CPET_HIP_TRY(hipGetLastError());
+    }
+  }
+
+  // With the chunk-lane form a workgroup need not fill its 64 slots, and where
+  // the batch is short of streamlines fewer slots let more workgroups share a
+  // frame: four assignments per workgroup, as long as the slots give each wave
+  // a task (see topo_run).  Two frames of 10,206 streamlines, 8,000 charges in
+  // the mean: 32 -> 26 ms with 20 slots; eight frames of 10,648: 173 ms with
+  // 64, 182 with 48.
+  int slots = 64;
+  if (d_chunks) {
+    const int want = std::max((int)(Lt / (4LL * G0)), 64 / chunk_groups(chg_off[F] / F));
+    slots = std::max(4, std::min(64, (want + 3) / 4 * 4));
+  }
   // Assignments: frames by decreasing work, one entry per A streamlines.
   // A workgroup that takes an assignment runs its 64 slots on that frame
   // until the frame's queue is empty, then drains them; larger assignments
   // put fewer workgroups on a frame, each running more streamlines per slot,
   // so the drain is a smaller share of its work.  A grows from 64 to 256
-  // while the batch still gives every workgroup four or more assignments.
-  const int A = 64 * std::max(1, std::min(4, (int)(Lt / ((long long)G0 * 64 * 4))));
+  // (of 64 slots) while the batch still gives every workgroup four or more assignments.
+  const int A = slots * std::max(1, std::min(4, (int)(Lt / ((long long)G0 * 64 * 4))));
   std::vector<int> byc(F);
   for (int f = 0; f < F; ++f) byc[f] = f;
   std::sort(byc.begin(), byc.end(), [&](int a, int b) {
@@ -1700,6 +2054,8 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   ba.n_assign = (int)assign.size();
   ba.assign_counter = d_cnt + F;
   ba.far_unsafe = d_far_unsafe;
+  ba.chunks = d_chunks;
+  ba.slots = slots;
   if ((rc = prof_mark(ctx, 0))) return rc;
   if (d_far) {  // the far-form frames (none when every flag is set)
     switch (S) {
