@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "cpet_internal.h"
+#include "smallfield.h"
 
 namespace cpet {
 
@@ -524,14 +525,14 @@ int cpet_ctx_refined_points(cpet_ctx* ctx, long long* n) {
     return CPET_ERR_ARG;
   }
   std::lock_guard<std::mutex> lk(ctx->mu);
-  *n = 0;
+  *n = ctx->all_f64;
   if (!ctx->fix_count) return CPET_OK;
   int rc = ctx_activate(ctx);
   if (rc) return rc;
   int v = 0;
   CPET_HIP_TRY(hipMemcpyAsync(&v, ctx->fix_count, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   CPET_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  *n = v;
+  *n += v;
   return CPET_OK;
 }
 
@@ -572,8 +573,20 @@ static int field_common(cpet_ctx* ctx, bool grid_mode, int nx, int ny, int nz,
   const float4* ch = nullptr;
   const double4* chd = nullptr;
   int npad = 0;
-  rc = pack_charges(ctx, N, x, q, dev, &ch, &chd, &npad);
-  if (rc) return rc;
+  const int kind = grid_mode ? 0 : 1;
+  // few pairs in the default precision and output type, with no launch shape
+  // asked for: one launch, straight from the caller's arrays
+  const bool small = (flags & CPET_F_PREC_MASK) == 0 && !(flags & CPET_F_OUT_F64) &&
+                     !(E_out && phi_out && !soften) && ctx->tune[kind][0] <= 0 &&
+                     ctx->tune[kind][1] <= 0 && small_field_ok(grid_mode, M, N);
+  const void *dx = nullptr, *dq = nullptr;
+  if (small) {
+    if ((rc = stage_in(ctx, kSlotX, x, (size_t)N * 3 * sizeof(float), dev, &dx))) return rc;
+    if ((rc = stage_in(ctx, kSlotQ, q, (size_t)N * sizeof(float), dev, &dq))) return rc;
+  } else {
+    rc = pack_charges(ctx, N, x, q, dev, &ch, &chd, &npad);
+    if (rc) return rc;
+  }
   const void *dax = nullptr, *day = nullptr, *daz = nullptr, *dpts = nullptr;
   if (grid_mode) {
     void* axes = nullptr;
@@ -608,8 +621,14 @@ static int field_common(cpet_ctx* ctx, bool grid_mode, int nx, int ny, int nz,
       if (rc) return rc;
     }
   }
-  const int kind = grid_mode ? 0 : 1;
-  rc = field_launch(ctx, grid_mode, nx, ny, nz, (const float*)dax,
+  ctx->all_f64 = 0;
+  if (small)
+    rc = small_field_launch(ctx, ny, nz, (const float*)dax, (const float*)day,
+                            (const float*)daz, M, (const float*)dpts, N, (const float*)dx,
+                            (const float*)dq, E_out ? (float*)dE : nullptr,
+                            phi_out ? (float*)dphi : nullptr, soften != 0);
+  else
+    rc = field_launch(ctx, grid_mode, nx, ny, nz, (const float*)dax,
                     (const float*)day, (const float*)daz, M,
                     (const float*)dpts, ch, chd, npad, E_out ? dE : nullptr,
                     phi_out ? dphi : nullptr, soften, flags, ctx->tune[kind][0],

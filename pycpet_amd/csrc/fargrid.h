@@ -18,13 +18,12 @@ struct FarGrid {
 };
 
 // Axes shorter than the 12 nodes by more than a third would sum at more nodes
-// than points.  The launches and node sums cost at least 60 us, which the
-// direct kernel takes at about 1e8 point-charge pairs: 41^3 x 1k (7e7 pairs)
-// 54 us direct, 41^3 x 4k (2.8e8) 150 us direct and 90 us here.  In a batch
+// than points.  The launches and node sums cost 35 to 70 us, which the one-launch
+// path takes at 5e7 point-charge pairs (smallfield.h has both sides).  In a batch
 // the launches are shared, and the direct kernel has no charge split: a 21^3 x
 // 40k frame alone keeps it busy for 1.5 ms.
 constexpr int kFarMinAxis = 8;
-constexpr double kFarMinPairs = 2e8;
+constexpr double kFarMinPairs = 5e7;
 constexpr double kFarMinPairsBatch = 2e7;
 
 // Whether an nx x ny x nz grid of npad (padded) charges takes the

@@ -45,6 +45,7 @@
 
 #include "cpet_internal.h"
 #include "fargrid.h"
+#include "smallfield.h"
 
 namespace cpet {
 namespace {
@@ -1028,6 +1029,8 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   std::vector<int32_t> geo(4 * (size_t)F), ax_off(F), blk;
   std::vector<int64_t> out_off(F);
   std::vector<FarGrid> fars;  // frames of the interpolating path, as field_launch chooses
+  std::vector<int> smalls;    // frames of the FP64 pair terms (smallfield.hip)
+  long long small_pts = 0;
   const bool may_far = mode == kModeAuto && !(flags & CPET_F_OUT_F64) && ctx->tune[4][0] <= 0;
   const int ch_total = chg_off.empty() ? 0 : chg_off.back();
   long long pts = 0;
@@ -1054,13 +1057,29 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
                              npad, chg_off[f], out_off[f]});
       continue;
     }
+    const long long M = (long long)nx * ny * nz;
+    if (may_far && !(E_out && phi_out && !soften) && small_field_ok(true, M, npad)) {
+      smalls.push_back(f);
+      small_pts += M;
+      continue;
+    }
     const long long lanes = (long long)nx * ny * nzc;
     for (long long b = 0; b < (lanes + 255) / 256; ++b) {
       blk.push_back(f);
       blk.push_back((int32_t)b);
     }
   }
+  const int nblk = (int)(blk.size() / 2);
+  const int P = small_field_points(ctx, small_pts);
+  for (int f : smalls) {
+    const long long M = (long long)geo[4 * f] * geo[4 * f + 1] * geo[4 * f + 2];
+    for (int b = 0; b < (M + P - 1) / P; ++b) {
+      blk.push_back(f);
+      blk.push_back(b);
+    }
+  }
   ctx->fix_count = nullptr;
+  ctx->all_f64 = E_out ? small_pts : 0;
   int rc = prof_mark(ctx, 0);
   if (rc) return rc;
   if (!fars.empty()) {
@@ -1099,6 +1118,18 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   a.fix_count = nullptr;
   a.fix_list = nullptr;
   a.near = nullptr;
+  if (!smalls.empty()) {
+    const SmallBatch sb = {a.blk + 2 * (size_t)nblk, a.geo, a.ax_off, a.out_off, a.chg_off, a.axes,
+                           ch};
+    if ((rc = small_batch_launch(ctx, P, (int)(blk.size() / 2) - nblk, sb, (float*)E_out,
+                                 (float*)phi_out, soften != 0)))
+      return rc;
+    if (!nblk) {
+      for (int i = 1; i < 3; ++i)
+        if ((rc = prof_mark(ctx, i))) return rc;
+      return CPET_OK;
+    }
+  }
   if (what == kWhatESoft && ch_total > 0) {
     void* nf = nullptr;
     if ((rc = ctx_buf(ctx, kSlotNear, (size_t)F * sizeof(int), &nf))) return rc;
@@ -1110,7 +1141,6 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   }
   const bool check = mode == kModeAuto && E_out != nullptr;
   if (check && (rc = fix_prepare(ctx, pts, &a.fix_count, &a.fix_list))) return rc;
-  const int nblk = (int)(blk.size() / 2);
   bool ok = false;
   switch (what) {
     case kWhatESoft: ok = launch_batch_w<kWhatESoft>(mode, K, st, nblk, ch, chd, a); break;
