@@ -401,6 +401,13 @@ int cpet_order_stats(cpet_ctx *ctx, int64_t n, int cols, const double *x, int n_
                      const int32_t *sel_cols, const int64_t *sel_ranks, double *values,
                      int64_t *nan_counts, uint32_t flags);
 
+/* Copies n host arrays, src[i] of bytes[i] bytes, one behind the other to the
+ * device memory at dst, on the context's stream.  The arrays may be reused
+ * when a later call on the context has waited for the stream.  No counterpart
+ * in the reference. */
+int cpet_upload_rows(cpet_ctx *ctx, int n, const void *const *src, const int64_t *bytes,
+                     void *dst);
+
 /* out (F,F) double: out[i][j] = sum over bins with h_i + h_j != 0 of
  * (h_i - h_j)^2 / (h_i + h_j), halved; zero diagonal.  Replaces
  * distance_numpy + construct_distance_matrix (CPET/utils/calculator.py:

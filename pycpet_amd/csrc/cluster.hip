@@ -316,6 +316,29 @@ int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const 
   return CPET_OK;
 }
 
+int cpet_upload_rows(cpet_ctx* ctx, int n, const void* const* src, const int64_t* bytes,
+                     void* dst) {
+  if (!ctx || n < 0 || (n > 0 && (!src || !bytes || !dst))) {
+    set_error("cpet_upload_rows: bad arguments");
+    return CPET_ERR_ARG;
+  }
+  for (int i = 0; i < n; ++i)
+    if (bytes[i] < 0 || (bytes[i] > 0 && !src[i])) {
+      set_error("cpet_upload_rows: array %d is NULL or of negative size", i);
+      return CPET_ERR_ARG;
+    }
+  std::lock_guard<std::mutex> lk(ctx->mu);
+  const int rc = ctx_activate(ctx);
+  if (rc) return rc;
+  char* to = (char*)dst;
+  for (int i = 0; i < n; ++i) {
+    if (bytes[i])
+      CPET_HIP_TRY(hipMemcpyAsync(to, src[i], (size_t)bytes[i], hipMemcpyHostToDevice, ctx->stream));
+    to += bytes[i];
+  }
+  return CPET_OK;
+}
+
 int cpet_order_stats(cpet_ctx* ctx, int64_t n, int cols, const double* x, int n_sel,
                      const int32_t* sel_cols, const int64_t* sel_ranks, double* values,
                      int64_t* nan_counts, uint32_t flags) {

@@ -259,3 +259,23 @@ def test_make_histograms_mem_files(gpu_ctx, oracle_mod, tmp_path):
     m = CH.construct_distance_matrix_mem(paths, ctx=gpu_ctx)
     np.testing.assert_allclose(m, oracle_mod.chi2_matrix_mem(list(want)), rtol=1e-12, atol=1e-15)
     assert np.all(np.diag(m) == 0.0)
+
+
+def test_rows_uploaded_frame_by_frame(gpu_ctx):
+    """Frames that lie anywhere in memory (a view, a transposed array, float32,
+    lists, no rows) land behind one another: counts equal numpy's."""
+    from pycpet_amd import clusterhist as CH
+
+    rng = np.random.default_rng(12)
+    big = np.abs(rng.normal(1.0, 0.4, (700, 2)))
+    frames = [big[:300], big[300:301], np.zeros((0, 2)), np.asfortranarray(big[301:500]),
+              big[500:].astype(np.float32), big[::-3].tolist()]
+    ed, ec = np.linspace(0, 3, 14), np.linspace(0, 3, 8)
+    hist = CH.histograms_from_features(frames, edges=(ed, ec), ctx=gpu_ctx)
+    for f, h in zip(frames, hist):
+        f = np.asarray(f, np.float64).reshape(-1, 2)
+        want = np.histogram2d(f[:, 0], f[:, 1], bins=[ed, ec])[0].ravel()
+        if len(f):
+            np.testing.assert_array_equal(h, want / want.sum())
+        else:
+            assert np.isnan(h).all()
