@@ -214,3 +214,25 @@ def test_autotuned_batch_shape(gpu_ctx):
         assert AT.tune_batch_topo(gpu_ctx, frames, cache=cache) == (S, G)
     finally:
         gpu_ctx.set_tuning(3, 0, 0)
+
+
+def test_batch_order_within_and_across_frames(gpu_ctx):
+    """The longest-first order counts in LDS where a workgroup's 1,024
+    streamlines are of one frame and one by one where they are not: frames of
+    one streamline, of just under, at and over a workgroup's share, with most
+    step limits alike."""
+    from pycpet_amd import batch, ops
+    from pycpet_amd import workloads as W
+
+    d = np.array([0.6, 0.5, 0.55], np.float32)
+    for n_charges in (12, 300):  # one-wave and 16-wave workgroups
+        x, q = W.ball_exclusion(n_charges, 12.0, 0.6, 1.5, seed=9)
+        frames = []
+        for i, L in enumerate((1, 1023, 1024, 5000, 30, 2049)):
+            st, it, _ = W.topo_starts(L, d, 0.01, 20, seed=60 + i, start_seed=70 + i)
+            frames.append({"x": x, "q": q, "starts": st, "n_iter": it, "h": 0.01, "dims": d})
+        for f, r in zip(frames, batch.batch_topo(frames, ctx=gpu_ctx)):
+            a = ops.topo(f["starts"], f["n_iter"], f["h"], f["dims"], f["x"], f["q"], ctx=gpu_ctx)
+            np.testing.assert_array_equal(r.feats, a.feats)
+            np.testing.assert_array_equal(r.steps, a.steps)
+            np.testing.assert_array_equal(r.exited, a.exited)
