@@ -623,6 +623,7 @@ def main() -> int:
             "kernel_ms": float(np.mean(kms)),  # field kernel + charge-split reduction
             "recompute_ms": float(np.mean(fms)),
             "recomputed_points": ctx.refined_points(),
+            # of the direct sum's pairs, most of which are interpolated
             "achieved_tflops": FLOP_PER_PAIR * vpairs / (np.mean(kms) * 1e-3) / 1e12,
         }
         # the same grid, potential only (volume_ESP): mixed FP32/FP64 pair
@@ -642,6 +643,7 @@ def main() -> int:
             "pair_evals_per_s": vpairs / pwall,
             "ms_per_frame": 1e3 * pwall,
             "kernel_ms": float(np.mean(kms)),
+            # as above
             "achieved_tflops": 11 * vpairs / (np.mean(kms) * 1e-3) / 1e12,
         }
 
