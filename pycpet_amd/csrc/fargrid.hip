@@ -49,6 +49,9 @@ constexpr int kMaxHalvings = 4;        // per axis: grids of up to 432 points
 constexpr int kMaxLevels = kMaxHalvings + 1;
 constexpr int kMaxAxis = kLeafMax << kMaxHalvings;
 constexpr int kMaxSegs = 2048;         // 64-charge segments: up to 131,072 charges
+constexpr int kTableBlocks = 2;        // classification workgroups per axis's tables
+constexpr int kClassWaves = 8;         // waves that share a segment's cells
+constexpr int kClassThreads = 64 * kClassWaves;
 constexpr int kThirds = 3;             // node workgroups per (cell, split)
 constexpr int kNodeLanes = 192;        // 48 node lines x 4 threads of 3 nodes
 constexpr int kNodeGroups = 4;         // that split a workgroup's charges
@@ -193,38 +196,68 @@ __device__ __forceinline__ void lagrange(double t, double* __restrict__ w) {
 
 // ---- extents and weights --------------------------------------------------
 
-// Centre and half width of every interval of one axis (level by level); x (n)
-// and the results in LDS.  An interval that holds a value that is not finite
-// is infinitely wide (its centre not a number): no charge is far from it.
-// Called by a whole workgroup; the same result wherever it is computed.
-__device__ __forceinline__ void axis_extents(const float* x, int n, int l, double* m, double* a) {
-  for (int e = threadIdx.x; e < (2 << l) - 1; e += blockDim.x) {
-    const int k = 31 - __clz(e + 1), t = e + 1 - (1 << k);
-    const int i1 = part_begin(n, k, t + 1);
+// Centre and half width of every interval (level by level) of the axes that x
+// (per axis, in LDS; null: left out) holds, into m and a (3 x kGeoPerAxis, LDS).
+// An interval that holds a value that is not finite is infinitely wide (its
+// centre not a number): no charge is far from it.  Called by a whole workgroup; the
+// same result wherever it is computed.  The values are read once, by a lane per leaf
+// interval of any axis, and the coarser intervals join their halves.
+__device__ __forceinline__ void axis_extents(const float* const (&x)[3], Frame& f, double* m,
+                                             double* a) {
+  const int l = max(f.l[0], max(f.l[1], f.l[2]));
+  for (int e = threadIdx.x; e < 3 << l; e += kClassThreads) {
+    const int axis = e >> l, t = e & ((1 << l) - 1);
+    if (!x[axis] || t >> f.l[axis]) continue;
+    const int n = f.n[axis], k = f.l[axis], i1 = part_begin(n, k, t + 1);
+    const float* v = x[axis];
     float lo = INFINITY, hi = -INFINITY, sum = 0.f;
 #pragma unroll 4
     for (int i = part_begin(n, k, t); i < i1; ++i) {
-      lo = fminf(lo, x[i]);
-      hi = fmaxf(hi, x[i]);
-      sum += 0.f * x[i];  // not a number for a value that is not finite
+      lo = fminf(lo, v[i]);
+      hi = fmaxf(hi, v[i]);
+      sum += 0.f * v[i];  // not a number for a value that is not finite
     }
-    const bool fine = sum == 0.f;
-    m[e] = fine ? 0.5 * ((double)lo + (double)hi) : (double)NAN;
-    a[e] = fine ? fmax(0.5 * ((double)hi - (double)lo), 1e-12) : (double)INFINITY;
+    const int at = axis * kGeoPerAxis + (1 << k) - 1 + t;
+    m[at] = sum == 0.f ? (double)lo : (double)NAN;
+    a[at] = (double)hi;
   }
+  __syncthreads();
+  for (int k = l - 1; k >= 0; --k) {
+    for (int e = threadIdx.x; e < 3 << k; e += kClassThreads) {
+      const int axis = e >> k, t = e & ((1 << k) - 1);
+      if (!x[axis] || k >= f.l[axis]) continue;
+      const int at = axis * kGeoPerAxis + (1 << k) - 1 + t;
+      const int half = axis * kGeoPerAxis + (2 << k) - 1 + 2 * t;  // of two
+      const double lo0 = m[half], lo1 = m[half + 1];
+      m[at] = lo0 != lo0 || lo1 != lo1 ? (double)NAN : fmin(lo0, lo1);
+      a[at] = fmax(a[half], a[half + 1]);
+    }
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < 3 * kGeoPerAxis; e += kClassThreads) {
+    const int axis = e / kGeoPerAxis;
+    if (!x[axis] || e - axis * kGeoPerAxis >= (2 << f.l[axis]) - 1) continue;
+    const double lo = m[e], hi = a[e];
+    const bool fine = lo == lo;
+    m[e] = fine ? 0.5 * (lo + hi) : (double)NAN;
+    a[e] = fine ? fmax(0.5 * (hi - lo), 1e-12) : (double)INFINITY;
+  }
+  __syncthreads();
 }
 
 // One axis: extents to memory, the weights of its values at every level and
 // the ancestors' weights at the leaf intervals' nodes.
-__device__ void axis_tables(const FarArgs& A, Frame& f, int axis, const float* x,
+// Shared by kTableBlocks workgroups: a row is 12 FP64 divisions.
+__device__ void axis_tables(const FarArgs& A, Frame& f, int axis, int share, const float* x,
                             const double* m, const double* a) {
   const int n = f.n[axis], l = f.l[axis];
+  const int first = share * kClassThreads + threadIdx.x, stride = kClassThreads * kTableBlocks;
   double* geo = A.geo + f.geo0 + (long long)axis * kGeoPerAxis * 2;
-  for (int e = threadIdx.x; e < (2 << l) - 1; e += blockDim.x) {
+  for (int e = first; e < (2 << l) - 1; e += stride) {
     geo[2 * e] = m[e];
     geo[2 * e + 1] = a[e];
   }
-  for (int r = threadIdx.x; r < (l + 1) * n; r += blockDim.x) {
+  for (int r = first; r < (l + 1) * n; r += stride) {
     const int k = r / n, i = r - k * n;
     int t = (int)(((long long)i << k) / n);  // the part that holds value i, or one off
     while (t > 0 && i < part_begin(n, k, t)) --t;
@@ -233,7 +266,7 @@ __device__ void axis_tables(const FarArgs& A, Frame& f, int axis, const float* x
     lagrange(((double)x[i] - m[e]) / a[e], A.lag + f.lag0[axis] + (long long)r * kP);
   }
   const int rows = (1 << l) * l * kP;
-  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
+  for (int r = first; r < rows; r += stride) {
     const int j = r % kP, k = (r / kP) % l, t = r / (kP * l);
     const int e = (1 << l) - 1 + t, anc = (1 << k) - 1 + (t >> (l - k));
     const double X = fma(a[e], kNodeX[j], m[e]);
@@ -261,36 +294,44 @@ __device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], c
   return ok;
 }
 
-// One wave per 64 charges: the far mask of every cell (far from it, near all
+// One workgroup per 64 charges, its waves sharing the cells of a level (a cell is a
+// chain of some 1,000 cycles; one wave for all 73 cells of a 101^3 grid took 36
+// us, eight take 11): the far mask of every cell (far from it, near all
 // its ancestors) and the near mask of every leaf, so that each charge is in
 // exactly one mask of every leaf's path.  A cell whose parent is near none
 // of the wave's charges is skipped.  Padding is in no mask.  The frame's last
-// three workgroups make the tables of one axis each.
-__global__ __launch_bounds__(64) void far_classify_kernel(FarArgs A) {
+// workgroups make the tables, kTableBlocks those of one axis.
+__global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) {
   extern __shared__ char dyn[];
   Frame& f = frame_of_block(&FarFrame::class_blk0, blockIdx.x);
   const int b = blockIdx.x - f.class_blk0;
-  float* sx = (float*)dyn;                           // the widest axis
-  const int wide = max(f.n[0], max(f.n[1], f.n[2]));
-  double* sm = (double*)(dyn + ((wide * 4 + 15) & ~15));  // 3 x kGeoPerAxis
+  float* sx = (float*)dyn;  // the axes
+  const int values = f.n[0] + f.n[1] + f.n[2];
+  double* sm = (double*)(dyn + ((values * 4 + 15) & ~15));  // 3 x kGeoPerAxis
   double* sa = sm + 3 * kGeoPerAxis;
   unsigned long long* far = (unsigned long long*)(sa + 3 * kGeoPerAxis);  // cells
   unsigned long long* near = far + f.cells;                               // cells
-  const int lane = threadIdx.x;
-  const int only = b < f.nseg ? -1 : b - f.nseg;  // table workgroups: their axis
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int only = b < f.nseg ? -1 : (b - f.nseg) / kTableBlocks;  // table workgroups: their axis
   float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
   if (only < 0) c = A.ch[f.ch0 + (long long)b * 64 + lane];
+  const float* axes[3];
+  float* to = sx;
+#pragma unroll
   for (int i = 0; i < 3; ++i) {
-    if (only >= 0 && i != only) continue;
     const float* __restrict__ x = A.ax[i] + f.ax0[i];
-    __syncthreads();
-    for (int k = lane; k < f.n[i]; k += 64) sx[k] = x[k];
-    __syncthreads();
-    axis_extents(sx, f.n[i], f.l[i], sm + i * kGeoPerAxis, sa + i * kGeoPerAxis);
+    const bool used = only < 0 || i == only;
+    if (used)
+      for (int k = threadIdx.x; k < f.n[i]; k += kClassThreads) to[k] = x[k];
+    axes[i] = used ? to : nullptr;
+    to += f.n[i];
   }
   __syncthreads();
+  axis_extents(axes, f, sm, sa);
   if (only >= 0) {
-    axis_tables(A, f, only, sx, sm + only * kGeoPerAxis, sa + only * kGeoPerAxis);
+    axis_tables(A, f, only, (b - f.nseg) % kTableBlocks,
+                only == 0 ? axes[0] : only == 1 ? axes[1] : axes[2], sm + only * kGeoPerAxis,
+                sa + only * kGeoPerAxis);
     return;
   }
   const bool real = !(c.x == kPadCoord && c.y == kPadCoord && c.z == kPadCoord && c.w == 0.f);
@@ -298,7 +339,7 @@ __global__ __launch_bounds__(64) void far_classify_kernel(FarArgs A) {
   int cell0 = 0, parent0 = 0;
   for (int level = 0; level < f.levels; ++level) {
     const int cells = cells_at(f, level);
-    for (int k = 0; k < cells; ++k) {
+    for (int k = wave; k < cells; k += kClassWaves) {
       int t[3];
       cell_parts(f, level, k, t);
       const unsigned long long pm =
@@ -325,8 +366,8 @@ __global__ __launch_bounds__(64) void far_classify_kernel(FarArgs A) {
   }
   const int leaves = cell0 - parent0;
   unsigned long long* out = A.mask + f.mask0 + b;
-  for (int k = lane; k < f.cells; k += 64) out[(long long)k * f.nseg] = far[k];
-  for (int k = lane; k < leaves; k += 64)
+  for (int k = threadIdx.x; k < f.cells; k += kClassThreads) out[(long long)k * f.nseg] = far[k];
+  for (int k = threadIdx.x; k < leaves; k += kClassThreads)
     out[(long long)(f.cells + k) * f.nseg] = near[parent0 + k];
 }
 
@@ -787,7 +828,7 @@ struct Blocks {
 template <bool E, bool PHI>
 void far_launch(hipStream_t st, const FarArgs& A, const Blocks& n, bool soft) {
   constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
-  hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(64), n.lds, st, A);
+  hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(kClassThreads), n.lds, st, A);
   hipLaunchKernelGGL((far_nodes_kernel<E, PHI>), dim3((unsigned)n.nodes), dim3(kNodeThreads), 0, st,
                      A);
   if (n.reduce)
@@ -836,13 +877,13 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
     while (done < F) {
       const FarGrid& g = grids[done];
       FarFrame f = {};
-      int wide = 0;
+      int values = 0;
       for (int i = 0; i < 3; ++i) {
         f.n[i] = g.n[i];
         f.l[i] = halvings(g.n[i]);
         f.ax0[i] = g.ax0[i];
         f.levels = std::max(f.levels, f.l[i] + 1);
-        wide = std::max(wide, g.n[i]);
+        values += g.n[i];
       }
       f.nseg = g.npad / 64;
       f.ch0 = g.ch0;
@@ -885,11 +926,11 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
       mask += mk;
       near += nr;
       geo += 3LL * kGeoPerAxis * 2;
-      n.classify += f.nseg + 3;
+      n.classify += f.nseg + 3 * kTableBlocks;
       n.nodes += nb + leaves;
       n.reduce += rb;
       n.eval += leaves * f.xblocks;
-      n.lds = std::max(n.lds, (size_t)((wide * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
+      n.lds = std::max(n.lds, (size_t)((values * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
                                   (size_t)f.cells * 16);
       fr.push_back(f);
       ++done;
