@@ -38,6 +38,7 @@
 
 #include "cpet_internal.h"
 #include "fargrid.h"
+#include "pairterm.h"
 
 namespace cpet {
 namespace {
@@ -613,16 +614,6 @@ __global__ __launch_bounds__(kRedThreads) void far_reduce_kernel(FarArgs A) {
 
 // ---- points --------------------------------------------------------------------
 
-// 1 / r as the direct kernels' potential has it: +inf at r = 0, not a number
-// at r = inf; ye is the field's, which is 0 there (FP32 rsq).
-__device__ __forceinline__ double near_rsqrt(double r2, double& ye) {
-  const double y = (double)__builtin_amdgcn_rsqf((float)r2);
-  const double e = fma(-r2, fmin(y * y, 1.7976931348623157e308), 1.0);
-  const double v = fma(0.5 * y, e, y);
-  ye = y == 0.0 ? 0.0 : v;
-  return v;
-}
-
 template <bool E, bool PHI, bool SOFT>
 __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kernel(FarArgs A) {
   constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
@@ -744,7 +735,7 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
   const float* __restrict__ ay = A.ax[1] + f.ax0[1];
   const float* __restrict__ az = A.ax[2] + f.ax0[2];
   double rclamp;
-  near_rsqrt((double)1e-6f, rclamp);
+  pair_rsqrt((double)1e-6f, rclamp);
   const int chunks = (n[2] + K - 1) / K, items = np * n[1] * chunks;
   for (int i0 = 0; i0 < items; i0 += kEvalThreads) {  // the same rounds for every thread
     const int i = min(i0 + tid, items - 1);
@@ -786,10 +777,10 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
         for (int k = 0; k < K; ++k) {
           const double dz = pz[k] - c.z;
           double ye;
-          const double y = near_rsqrt(fma(dz, dz, dxy2), ye);
+          const double y = pair_rsqrt(fma(dz, dz, dxy2), ye);
           if constexpr (PHI) acc[k][C - 1] = fma(c.w, y, acc[k][C - 1]);
           if constexpr (E) {
-            const double re = SOFT ? fmin(ye, rclamp) : ye;
+            const double re = pair_floor<SOFT, !PHI>(ye, rclamp);
             const double w = (c.w * re) * (re * re);
             acc[k][0] = fma(w, dx, acc[k][0]);
             acc[k][1] = fma(w, dy, acc[k][1]);

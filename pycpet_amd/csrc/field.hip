@@ -45,6 +45,7 @@
 
 #include "cpet_internal.h"
 #include "fargrid.h"
+#include "pairterm.h"
 #include "smallfield.h"
 
 namespace cpet {
@@ -79,16 +80,7 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
   return (x == 0.0) ? y : y1;
 }
 
-// One Newton-Raphson step in FP64 from an FP32 estimate of 1/sqrt(x):
-// relative error ~1e-7 -> ~1e-14.  Clamping y*y keeps x == 0 (y = +inf)
-// from producing 0*inf: the residual is then 1 and the result stays +inf.
-__device__ __forceinline__ double rsqrt_refine(float seed, double x) {
-  const double y = (double)seed;
-  const double e = fma(-x, fmin(y * y, 1.7976931348623157e308), 1.0);
-  return fma(0.5 * y, e, y);
-}
-
-// The same step for x > 0 (no charge on the point): one clamp fewer.
+// rsqrt_refine's step for x > 0 (no charge on the point): one clamp fewer.
 __device__ __forceinline__ double rsqrt_refine_pos(float seed, double x) {
   const double y = (double)seed;
   const double e = fma(-x, y * y, 1.0);

@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "cpet_internal.h"
+#include "pairterm.h"
 #include "smallfield.h"
 
 namespace cpet {
@@ -42,16 +43,6 @@ struct SmallArgs {
   const float *x, *q;       // (N,3), (N)
   float *e, *phi;           // (M,3), (M)
 };
-
-// 1 / r for the potential (+inf at r = 0), and for the field, where a charge
-// beyond the FP32 range of r^2 adds 0 (as an FP32 rsq of inf does).
-__device__ __forceinline__ double pair_rsqrt(double r2, double& ye) {
-  const double y = (double)__builtin_amdgcn_rsqf((float)r2);
-  const double e = fma(-r2, fmin(y * y, 1.7976931348623157e308), 1.0);
-  const double v = fma(0.5 * y, e, y);
-  ye = y == 0.0 ? 0.0 : v;
-  return v;
-}
 
 // P points per workgroup: thread t has point t % P and every (1024 / P)-th
 // charge from t / P on.
@@ -103,11 +94,7 @@ __global__ __launch_bounds__(kThreads) void small_field_kernel(SmallArgs a) {
     const double y = pair_rsqrt(fma(dz, dz, fma(dy, dy, dx * dx)), ye);
     if constexpr (PHI) acc[C - 1] = fma(q, y, acc[C - 1]);
     if constexpr (E) {
-      // 1 / r of a coordinate that is not a number: kept for E alone on a grid,
-      // otherwise the floor's, as the direct kernels have it
-      const double re = !SOFT          ? ye
-                        : GRID && !PHI ? (ye > rclamp ? rclamp : ye)
-                                       : fmin(ye, rclamp);
+      const double re = pair_floor<SOFT, GRID && !PHI>(ye, rclamp);
       const double w = (q * re) * (re * re);
       acc[0] = fma(w, dx, acc[0]);
       acc[1] = fma(w, dy, acc[1]);

@@ -245,3 +245,44 @@ def test_captured_replays(gpu_ctx, batched):
         torch.cuda.synchronize()
         assert torch.equal(got, want)
     step.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["E", "E unsoftened", "phi"])
+def test_one_output_of_values_that_are_not_finite(gpu_ctx, what):
+    """E alone (with and without the floor) and phi alone of infinite and NaN charges and axis
+    values: the same components are NaN as in the direct kernel, the others agree.  E alone is
+    NaN in all three components for a NaN coordinate: no charge is within the floor's reach."""
+    from pycpet_amd import ops
+
+    axes, x, q = _frame(seed=6)
+    kw = {"want_E": what != "phi", "want_phi": what == "phi", "soften": what != "E unsoftened"}
+
+    def same():
+        far = [a for a in ops.field_grid(*axes, x, q, ctx=gpu_ctx, **kw) if a is not None][0]
+        gpu_ctx.set_tuning(0, 2, 0)
+        try:
+            direct = [a for a in ops.field_grid(*axes, x, q, ctx=gpu_ctx, **kw)
+                      if a is not None][0]
+        finally:
+            gpu_ctx.set_tuning(0, 0, 0)
+        np.testing.assert_array_equal(np.isnan(far), np.isnan(direct))
+        ok = np.isfinite(direct)
+        scale = np.sqrt(np.mean(direct[ok].astype(float) ** 2)) if ok.any() else 1.0
+        np.testing.assert_allclose(far[ok], direct[ok], rtol=1e-4, atol=1e-5 * scale)
+        return far
+
+    keep = x[0].copy()
+    for bad in (np.inf, np.nan):
+        for k in range(3):
+            x[0, k] = bad
+            far = same()
+            x[0] = keep
+            if np.isnan(bad):
+                assert np.isnan(far).all()
+        q0, q[0] = q[0], bad
+        same()
+        q[0] = q0
+        v, axes[1][4] = axes[1][4], bad
+        same()
+        axes[1][4] = v
