@@ -811,13 +811,18 @@ int halvings(int n) {
   return l;
 }
 
-struct Blocks {
+// Frames that share the four launches: workgroups of each, and the elements of
+// the scratch arrays in FarArgs.
+struct Group {
+  int first = 0, count = 0;  // of the call's frames
   long long classify = 0, nodes = 0, reduce = 0, eval = 0;
   size_t lds = 0;  // of the classification
+  long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, near = 0;
+  size_t bytes() const { return (size_t)(part + val + geo + lag + mask) * 8 + (size_t)near * 4; }
 };
 
 template <bool E, bool PHI>
-void far_launch(hipStream_t st, const FarArgs& A, const Blocks& n, bool soft) {
+void far_launch(hipStream_t st, const FarArgs& A, const Group& n, bool soft) {
   constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
   hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(kClassThreads), n.lds, st, A);
   hipLaunchKernelGGL((far_nodes_kernel<E, PHI>), dim3((unsigned)n.nodes), dim3(kNodeThreads), 0, st,
@@ -842,17 +847,21 @@ bool far_grid_ok(int nx, int ny, int nz, int npad, double min_pairs) {
   return npad <= 64 * kMaxSegs && (double)nx * ny * nz * npad >= min_pairs;
 }
 
-// Runs the frames in as few groups as the scratch bound allows.
+// Runs the frames in as few groups as the scratch bound allows.  All groups are
+// planned first: their frames are one table, uploaded at once, so that a call of
+// the same shapes finds it unchanged (and can be captured) whatever their number.
 int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const float* const (&ax)[3],
                     const float4* ch, bool want_e, bool want_phi, bool soft, void* e, void* phi) {
   const int C = (want_e ? 3 : 0) + (want_phi ? 1 : 0);
   constexpr size_t kMaxScratch = (size_t)1 << 30;
   const int F = (int)grids.size();
+  std::vector<FarFrame> frames;
+  std::vector<Group> groups;
+  size_t bytes = 0;
   int done = 0;
   while (done < F) {
-    std::vector<FarFrame> fr;
-    long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, near = 0;
-    Blocks n;
+    Group n;
+    n.first = done;
     // Node workgroups: two per CU over all frames, shared out by work.  A
     // level's far charges, over all its cells, are about the charges of the
     // frame (level 0) or twice that: with kRho, most charges of a level's
@@ -883,11 +892,11 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
       f.node_blk0 = (int)n.nodes;
       f.red_blk0 = (int)n.reduce;
       f.eval_blk0 = (int)n.eval;
-      f.part0 = part;
-      f.val0 = val;
-      f.geo0 = geo;
-      f.mask0 = mask;
-      f.near0 = near;
+      f.part0 = n.part;
+      f.val0 = n.val;
+      f.geo0 = n.geo;
+      f.mask0 = n.mask;
+      f.near0 = n.near;
       long long p = 0, nb = 0, rb = 0, leaves = 0;
       for (int k = 0; k < f.levels; ++k) {
         leaves = cells_at(f, k);
@@ -898,58 +907,60 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
         p += leaves * f.splits[k] * C * kNodes;
         rb += red_blocks((int)leaves, C, f.splits[k]);
       }
-      const long long v = (long long)f.cells * C * kNodes;
-      const long long mk = (f.cells + leaves) * f.nseg;
-      const long long nr = leaves * (64LL * f.nseg + 1);
-      if (!fr.empty() &&
-          (size_t)(part + p + val + v + mask + mk) * 8 + (size_t)(near + nr) * 4 > kMaxScratch)
-        break;
+      Group with = n;
+      for (int i = 0; i < 3; ++i) {
+        f.lag0[i] = with.lag;
+        with.lag += (long long)(f.l[i] + 1) * f.n[i] * kP;
+        f.tr0[i] = with.lag;
+        with.lag += (long long)(1 << f.l[i]) * f.l[i] * kP * kP;
+      }
+      with.part += p;
+      with.val += (long long)f.cells * C * kNodes;
+      with.mask += (f.cells + leaves) * f.nseg;
+      with.near += leaves * (64LL * f.nseg + 1);
+      with.geo += 3LL * kGeoPerAxis * 2;
+      if (n.count && with.bytes() > kMaxScratch) break;
       const int widest = (f.n[0] + (1 << f.l[0]) - 1) >> f.l[0];
       f.xblocks = (widest + kPlanes - 1) / kPlanes;
-      for (int i = 0; i < 3; ++i) {
-        f.lag0[i] = lag;
-        lag += (long long)(f.l[i] + 1) * f.n[i] * kP;
-        f.tr0[i] = lag;
-        lag += (long long)(1 << f.l[i]) * f.l[i] * kP * kP;
-      }
-      part += p;
-      val += v;
-      mask += mk;
-      near += nr;
-      geo += 3LL * kGeoPerAxis * 2;
-      n.classify += f.nseg + 3 * kTableBlocks;
-      n.nodes += nb + leaves;
-      n.reduce += rb;
-      n.eval += leaves * f.xblocks;
-      n.lds = std::max(n.lds, (size_t)((values * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
-                                  (size_t)f.cells * 16);
-      fr.push_back(f);
+      with.classify += f.nseg + 3 * kTableBlocks;
+      with.nodes += nb + leaves;
+      with.reduce += rb;
+      with.eval += leaves * f.xblocks;
+      with.lds = std::max(n.lds, (size_t)((values * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
+                                     (size_t)f.cells * 16);
+      ++with.count;
+      n = with;
+      frames.push_back(f);
       ++done;
     }
-    void* buf = nullptr;
-    int rc = ctx_buf(ctx, kSlotFarGrid, (size_t)(part + val + geo + lag + mask) * 8 + (size_t)near * 4, &buf);
-    if (rc) return rc;
+    bytes = std::max(bytes, n.bytes());
+    groups.push_back(n);
+  }
+  void *buf = nullptr, *tab = nullptr;
+  int rc = ctx_buf(ctx, kSlotFarGrid, bytes, &buf);
+  if (rc) return rc;
+  if (F > 1) {
+    if ((rc = ctx_buf(ctx, kSlotFarTables, F * sizeof(FarFrame), &tab))) return rc;
+    if ((rc = upload_table(ctx, kTabFarFrames, tab, frames.data(), F * sizeof(FarFrame))))
+      return rc;
+  }
+  for (const Group& n : groups) {
     FarArgs A = {};
-    A.F = (int)fr.size();
+    A.F = n.count;
     A.ch = ch;
     for (int i = 0; i < 3; ++i) A.ax[i] = ax[i];
     A.part = (double*)buf;
-    A.val = A.part + part;
-    A.geo = A.val + val;
-    A.lag = A.geo + geo;
-    A.mask = (unsigned long long*)(A.lag + lag);
-    A.near = (int*)(A.mask + mask);
+    A.val = A.part + n.part;
+    A.geo = A.val + n.val;
+    A.lag = A.geo + n.geo;
+    A.mask = (unsigned long long*)(A.lag + n.lag);
+    A.near = (int*)(A.mask + n.mask);
     A.e = e;
     A.phi = phi;
-    if (A.F == 1) {
-      A.one = fr[0];
-    } else {
-      void* tab = nullptr;
-      if ((rc = ctx_buf(ctx, kSlotFarTables, fr.size() * sizeof(FarFrame), &tab))) return rc;
-      if ((rc = upload_table(ctx, kTabFarFrames, tab, fr.data(), fr.size() * sizeof(FarFrame))))
-        return rc;
-      A.frames = (const FarFrame*)tab;
-    }
+    if (n.count == 1)
+      A.one = frames[n.first];
+    else
+      A.frames = (const FarFrame*)tab + n.first;
     if (want_e && want_phi)
       far_launch<true, true>(ctx->stream, A, n, soft);
     else if (want_e)

@@ -286,3 +286,37 @@ def test_one_output_of_values_that_are_not_finite(gpu_ctx, what):
         v, axes[1][4] = axes[1][4], bad
         same()
         axes[1][4] = v
+
+
+@pytest.mark.gpu
+def test_captured_batch_of_several_scratch_groups(gpu_ctx):
+    """A batch whose node sums and near lists need more than the 1 GiB that one launch may take
+    (8 frames, 512 leaves each, 65,536 charges: 134 MB of near list a frame) runs in several; it
+    can be captured, its replays follow the inputs, and its frames equal the frames run alone
+    to one float32 rounding."""
+    import torch
+
+    from pycpet_amd import batch, graphs, ops
+
+    rng = np.random.default_rng(31)
+    T = lambda a: torch.from_numpy(a).cuda()
+    axis = T(np.linspace(-2.7, 2.7, 109).astype(np.float32))
+    fr = [{"axes": (axis, axis, axis),
+           "x": T(rng.uniform(-40, 40, (65536, 3)).astype(np.float32)),
+           "q": T(rng.normal(0, 0.4, 65536).astype(np.float32))} for _ in range(8)]
+    fn = lambda ctx: torch.cat([E for E, _ in batch.batch_volume(fr, ctx=ctx)])
+    step = graphs.CapturedStep(fn)
+    for k in range(3):
+        fr[k]["x"].add_(0.05)
+        got = step.replay()
+        torch.cuda.synchronize()
+        want = fn(gpu_ctx)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    step.close()
+    M = 109 ** 3
+    for k in (0, 7):
+        one, _ = ops.field_grid(axis, axis, axis, fr[k]["x"], fr[k]["q"], ctx=gpu_ctx)
+        b = want[k * M:(k + 1) * M]
+        scale = float(one.double().square().mean().sqrt())
+        assert float((one - b).abs().max()) <= 1e-7 * scale + 5e-6 * float(one.abs().max())
