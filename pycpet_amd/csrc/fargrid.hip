@@ -734,8 +734,7 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
   const float* __restrict__ ax = A.ax[0] + f.ax0[0];
   const float* __restrict__ ay = A.ax[1] + f.ax0[1];
   const float* __restrict__ az = A.ax[2] + f.ax0[2];
-  double rclamp;
-  pair_rsqrt((double)1e-6f, rclamp);
+  const double rclamp = pair_clamp();
   const int chunks = (n[2] + K - 1) / K, items = np * n[1] * chunks;
   for (int i0 = 0; i0 < items; i0 += kEvalThreads) {  // the same rounds for every thread
     const int i = min(i0 + tid, items - 1);
@@ -776,11 +775,10 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           const double dz = pz[k] - c.z;
-          double ye;
-          const double y = pair_rsqrt(fma(dz, dz, dxy2), ye);
+          double re;
+          const double y = pair_rsqrt<SOFT, !PHI>(fma(dz, dz, dxy2), rclamp, re);
           if constexpr (PHI) acc[k][C - 1] = fma(c.w, y, acc[k][C - 1]);
           if constexpr (E) {
-            const double re = pair_floor<SOFT, !PHI>(ye, rclamp);
             const double w = (c.w * re) * (re * re);
             acc[k][0] = fma(w, dx, acc[k][0]);
             acc[k][1] = fma(w, dy, acc[k][1]);

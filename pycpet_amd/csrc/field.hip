@@ -80,13 +80,6 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
   return (x == 0.0) ? y : y1;
 }
 
-// rsqrt_refine's step for x > 0 (no charge on the point): one clamp fewer.
-__device__ __forceinline__ double rsqrt_refine_pos(float seed, double x) {
-  const double y = (double)seed;
-  const double e = fma(-x, y * y, 1.0);
-  return fma(0.5 * y, e, y);
-}
-
 // Relative error target of the auto-mode check (see above): points whose
 // estimate u * A / |E| exceeds it are recomputed in FP64.
 constexpr double kAutoTol = 4e-6;

@@ -83,18 +83,17 @@ __global__ __launch_bounds__(kThreads) void small_field_kernel(SmallArgs a) {
     py = a.pts[3 * m + 1];
     pz = a.pts[3 * m + 2];
   }
-  double rclamp;
-  pair_rsqrt((double)1e-6f, rclamp);
+  const double rclamp = pair_clamp();
   double acc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) acc[c] = 0.0;
   auto pair = [&](double cx, double cy, double cz, double q) __attribute__((always_inline)) {
     const double dx = px - cx, dy = py - cy, dz = pz - cz;
-    double ye;
-    const double y = pair_rsqrt(fma(dz, dz, fma(dy, dy, dx * dx)), ye);
+    double re;
+    const double y =
+        pair_rsqrt<SOFT, GRID && !PHI>(fma(dz, dz, fma(dy, dy, dx * dx)), rclamp, re);
     if constexpr (PHI) acc[C - 1] = fma(q, y, acc[C - 1]);
     if constexpr (E) {
-      const double re = pair_floor<SOFT, GRID && !PHI>(ye, rclamp);
       const double w = (q * re) * (re * re);
       acc[0] = fma(w, dx, acc[0]);
       acc[1] = fma(w, dy, acc[1]);
