@@ -1,6 +1,7 @@
 // Grid field with the far charges interpolated (fargrid.hip).
 #pragma once
 
+#include <memory>
 #include <vector>
 
 #include "cpet_internal.h"
@@ -30,10 +31,16 @@ constexpr double kFarMinPairsBatch = 2e7;
 // interpolating path, from min_pairs (points x charges) on.
 bool far_grid_ok(int nx, int ny, int nz, int npad, double min_pairs);
 
-// Float32 E and / or phi of the grids (null: not wanted), queued on the
-// context's stream.  ax: the device arrays that hold the grids' x, y and z
-// axes.
-int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const float* const (&ax)[3],
-                    const float4* ch, bool want_e, bool want_phi, bool soft, void* e, void* phi);
+// The launches of some grids.  Null where their scratch cannot be had (memory has
+// run out, or the stream is being captured and they have not run on this context
+// before): the direct kernel takes them then.
+struct FarPlan;
+std::shared_ptr<const FarPlan> far_grid_plan(cpet_ctx* ctx, const std::vector<FarGrid>& grids,
+                                             bool want_e, bool want_phi);
+
+// Float32 E and / or phi (as planned) of the grids, queued on the context's
+// stream.  ax: the device arrays that hold the grids' x, y and z axes.
+int far_grid_run(cpet_ctx* ctx, const FarPlan& plan, const float* const (&ax)[3], const float4* ch,
+                 bool soft, void* e, void* phi);
 
 }  // namespace cpet

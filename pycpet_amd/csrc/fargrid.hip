@@ -107,6 +107,7 @@ struct FarFrame {
   long long tr0[3];    // per axis: leaf part x ancestor level x kP x kP
   long long mask0;     // (cells + leaves) x nseg: far masks, then the leaves' near masks
   long long near0;     // per leaf: number of near charges, then their numbers (64 nseg)
+  int leaf0;           // the launch's first leaf (see Group::range)
   long long out0;      // first output point
   long long ax0[3];    // first value of each axis
 };
@@ -469,8 +470,9 @@ __global__ __launch_bounds__(kNodeThreads, 6) void far_nodes_kernel(FarArgs A) {
     part += (long long)nb * C * kNodes;
     cell0 += cells;
   }
-  if (level == f.levels) {  // near list of leaf b
-    const unsigned long long* __restrict__ mask = A.mask + f.mask0 + (long long)(f.cells + b) * f.nseg;
+  if (level == f.levels) {  // the launch's b-th near list
+    const unsigned long long* __restrict__ mask =
+        A.mask + f.mask0 + (long long)(f.cells + f.leaf0 + b) * f.nseg;
     const int total = list_prefix<kNodeThreads>(mask, f.nseg, off, tmp);
     int* out = A.near + f.near0 + (long long)b * (64 * f.nseg + 1);
     if (tid == 0) out[0] = total;
@@ -621,7 +623,7 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
   constexpr int kPC = kPlanes * C;
   Frame& f = frame_of_block(&FarFrame::eval_blk0, blockIdx.x);
   const int b = blockIdx.x - f.eval_blk0;
-  const int leaf = b / f.xblocks, xb = b % f.xblocks;
+  const int list = b / f.xblocks, leaf = f.leaf0 + list, xb = b % f.xblocks;
   const int bottom = f.levels - 1;
   int t[3];
   cell_parts(f, bottom, leaf, t);
@@ -726,7 +728,7 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
     for (int k = 0; k < kP; ++k) s = fma(lagy[j * kP + k], w1[pc * kP * kP + k * kP + c], s);
     w2[(pc * kLeafMax + j) * kP + c] = s;
   }
-  const int* __restrict__ near = A.near + f.near0 + (long long)leaf * (64 * f.nseg + 1);
+  const int* __restrict__ near = A.near + f.near0 + (long long)list * (64 * f.nseg + 1);
   const float4* __restrict__ ch = A.ch + f.ch0;
   const int total = near[0];
   __syncthreads();
@@ -815,25 +817,43 @@ struct Group {
   int first = 0, count = 0;  // of the call's frames
   long long classify = 0, nodes = 0, reduce = 0, eval = 0;
   size_t lds = 0;  // of the classification
+  // Leaves whose near lists are held at once, of the leaves of one frame whose lists
+  // (room for every charge in each) would not fit the scratch bound; 0: all of them.
+  int range = 0, leaves = 0;
   long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, near = 0;
   size_t bytes() const { return (size_t)(part + val + geo + lag + mask) * 8 + (size_t)near * 4; }
 };
 
 template <bool E, bool PHI>
-void far_launch(hipStream_t st, const FarArgs& A, const Group& n, bool soft) {
+void far_launch(hipStream_t st, FarArgs A, const Group& n, bool soft) {
   constexpr int C = (E ? 3 : 0) + (PHI ? 1 : 0);
+  auto nodes = [&](long long blocks) {
+    hipLaunchKernelGGL((far_nodes_kernel<E, PHI>), dim3((unsigned)blocks), dim3(kNodeThreads), 0, st,
+                       A);
+  };
+  auto eval = [&](long long blocks) {
+    if (soft)
+      hipLaunchKernelGGL((far_eval_kernel<E, PHI, true>), dim3((unsigned)blocks),
+                         dim3(kEvalThreads), 0, st, A);
+    else
+      hipLaunchKernelGGL((far_eval_kernel<E, PHI, false>), dim3((unsigned)blocks),
+                         dim3(kEvalThreads), 0, st, A);
+  };
   hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(kClassThreads), n.lds, st, A);
-  hipLaunchKernelGGL((far_nodes_kernel<E, PHI>), dim3((unsigned)n.nodes), dim3(kNodeThreads), 0, st,
-                     A);
+  nodes(n.nodes);
   if (n.reduce)
     hipLaunchKernelGGL((far_reduce_kernel<C>), dim3((unsigned)n.reduce), dim3(kRedThreads), 0, st,
                        A);
-  if (soft)
-    hipLaunchKernelGGL((far_eval_kernel<E, PHI, true>), dim3((unsigned)n.eval), dim3(kEvalThreads),
-                       0, st, A);
-  else
-    hipLaunchKernelGGL((far_eval_kernel<E, PHI, false>), dim3((unsigned)n.eval),
-                       dim3(kEvalThreads), 0, st, A);
+  eval(n.eval);
+  // the other ranges of leaves: near lists alone (the workgroups behind those of
+  // the nodes), in the memory of the previous range's, and their points
+  if (n.range) A.one.node_blk0 = -(int)(n.nodes - n.range);
+  for (int left = n.leaves - n.range; n.range && left > 0; left -= n.range) {
+    A.one.leaf0 += n.range;
+    const int now = std::min(n.range, left);
+    nodes(now);
+    eval((long long)now * A.one.xblocks);
+  }
 }
 
 }  // namespace
@@ -845,16 +865,30 @@ bool far_grid_ok(int nx, int ny, int nz, int npad, double min_pairs) {
   return npad <= 64 * kMaxSegs && (double)nx * ny * nz * npad >= min_pairs;
 }
 
-// Runs the frames in as few groups as the scratch bound allows.  All groups are
-// planned first: their frames are one table, uploaded at once, so that a call of
-// the same shapes finds it unchanged (and can be captured) whatever their number.
-int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const float* const (&ax)[3],
-                    const float4* ch, bool want_e, bool want_phi, bool soft, void* e, void* phi) {
+struct FarPlan {
+  std::vector<FarFrame> frames;
+  std::vector<Group> groups;
+  bool want_e, want_phi;
+  void *buf = nullptr, *tab = nullptr;
+};
+
+// The frames in as few groups as the scratch bound allows.  The frames of all
+// groups are one table, uploaded at once, so that a call of the same shapes finds
+// it unchanged (and can be captured) whatever their number.
+//
+// The bound holds for one frame too: of the largest grid (4,681 cells) and charge
+// count, node sums, masks and tables take 0.7 GB, and near lists are held for as
+// many leaves at a time as the rest has room for (for all 4,096 they would take 2.1
+// GB).  217 x 218 x 217 points, 45,000 charges: two ranges of leaves.
+std::shared_ptr<const FarPlan> far_grid_plan(cpet_ctx* ctx, const std::vector<FarGrid>& grids,
+                                             bool want_e, bool want_phi) {
   const int C = (want_e ? 3 : 0) + (want_phi ? 1 : 0);
   constexpr size_t kMaxScratch = (size_t)1 << 30;
   const int F = (int)grids.size();
-  std::vector<FarFrame> frames;
-  std::vector<Group> groups;
+  auto plan = std::make_shared<FarPlan>();
+  plan->want_e = want_e;
+  plan->want_phi = want_phi;
+  std::vector<FarFrame>& frames = plan->frames;
   size_t bytes = 0;
   int done = 0;
   while (done < F) {
@@ -918,36 +952,51 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
       with.near += leaves * (64LL * f.nseg + 1);
       with.geo += 3LL * kGeoPerAxis * 2;
       if (n.count && with.bytes() > kMaxScratch) break;
+      long long lists = leaves;
+      if (with.bytes() > kMaxScratch) {  // a frame alone
+        const size_t list = (64 * (size_t)f.nseg + 1) * 4;
+        const size_t rest = with.bytes() - leaves * list;
+        lists = rest + list < kMaxScratch ? (long long)((kMaxScratch - rest) / list) : 1;
+        with.range = (int)lists;
+        with.leaves = (int)leaves;
+        with.near = lists * (64LL * f.nseg + 1);
+      }
       const int widest = (f.n[0] + (1 << f.l[0]) - 1) >> f.l[0];
       f.xblocks = (widest + kPlanes - 1) / kPlanes;
       with.classify += f.nseg + 3 * kTableBlocks;
-      with.nodes += nb + leaves;
+      with.nodes += nb + lists;
       with.reduce += rb;
-      with.eval += leaves * f.xblocks;
+      with.eval += lists * f.xblocks;
       with.lds = std::max(n.lds, (size_t)((values * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
                                      (size_t)f.cells * 16);
       ++with.count;
       n = with;
       frames.push_back(f);
       ++done;
+      if (n.range) break;
     }
     bytes = std::max(bytes, n.bytes());
-    groups.push_back(n);
+    plan->groups.push_back(n);
   }
-  void *buf = nullptr, *tab = nullptr;
-  int rc = ctx_buf(ctx, kSlotFarGrid, bytes, &buf);
-  if (rc) return rc;
-  if (F > 1) {
-    if ((rc = ctx_buf(ctx, kSlotFarTables, F * sizeof(FarFrame), &tab))) return rc;
-    if ((rc = upload_table(ctx, kTabFarFrames, tab, frames.data(), F * sizeof(FarFrame))))
-      return rc;
+  if (!(plan->buf = ctx_buf_try(ctx, kSlotFarGrid, bytes))) return nullptr;
+  if (F > 1 && !(plan->tab = ctx_buf_try(ctx, kSlotFarTables, F * sizeof(FarFrame))))
+    return nullptr;
+  return plan;
+}
+
+int far_grid_run(cpet_ctx* ctx, const FarPlan& plan, const float* const (&ax)[3], const float4* ch,
+                 bool soft, void* e, void* phi) {
+  if (plan.tab) {
+    const int rc = upload_table(ctx, kTabFarFrames, plan.tab, plan.frames.data(),
+                                plan.frames.size() * sizeof(FarFrame));
+    if (rc) return rc;
   }
-  for (const Group& n : groups) {
+  for (const Group& n : plan.groups) {
     FarArgs A = {};
     A.F = n.count;
     A.ch = ch;
     for (int i = 0; i < 3; ++i) A.ax[i] = ax[i];
-    A.part = (double*)buf;
+    A.part = (double*)plan.buf;
     A.val = A.part + n.part;
     A.geo = A.val + n.val;
     A.lag = A.geo + n.geo;
@@ -956,12 +1005,12 @@ int far_grid_launch(cpet_ctx* ctx, const std::vector<FarGrid>& grids, const floa
     A.e = e;
     A.phi = phi;
     if (n.count == 1)
-      A.one = frames[n.first];
+      A.one = plan.frames[n.first];
     else
-      A.frames = (const FarFrame*)tab + n.first;
-    if (want_e && want_phi)
+      A.frames = (const FarFrame*)plan.tab + n.first;
+    if (plan.want_e && plan.want_phi)
       far_launch<true, true>(ctx->stream, A, n, soft);
-    else if (want_e)
+    else if (plan.want_e)
       far_launch<true, false>(ctx->stream, A, n, soft);
     else
       far_launch<false, true>(ctx->stream, A, n, soft);

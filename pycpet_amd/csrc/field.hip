@@ -851,17 +851,17 @@ int field_launch(cpet_ctx* ctx, bool grid_mode, int nx, int ny, int nz,
   // 61 x 47 x 38 x 12k E 0.51 -> 0.085 ms.  The line: see kFarMinPairs.
   if (grid_mode && mode == kModeAuto && !(flags & CPET_F_OUT_F64) && forced_k <= 0 &&
       forced_splits <= 0 && far_grid_ok(nx, ny, nz, npad, kFarMinPairs)) {
-    ctx->fix_count = nullptr;
-    int rc = prof_mark(ctx, 0);
-    if (rc) return rc;
     const std::vector<FarGrid> g(1, FarGrid{{nx, ny, nz}, {0, 0, 0}, npad, 0, 0});
-    const float* const axes[3] = {ax, ay, az};
-    if ((rc = far_grid_launch(ctx, g, axes, ch, E_out != nullptr, phi_out != nullptr, soften != 0,
-                              E_out, phi_out)))
-      return rc;
-    for (int i = 1; i < 4; ++i)
-      if ((rc = prof_mark(ctx, i))) return rc;
-    return CPET_OK;
+    if (const auto plan = far_grid_plan(ctx, g, E_out != nullptr, phi_out != nullptr)) {
+      ctx->fix_count = nullptr;
+      int rc = prof_mark(ctx, 0);
+      if (rc) return rc;
+      const float* const axes[3] = {ax, ay, az};
+      if ((rc = far_grid_run(ctx, *plan, axes, ch, soften != 0, E_out, phi_out))) return rc;
+      for (int i = 1; i < 4; ++i)
+        if ((rc = prof_mark(ctx, i))) return rc;
+      return CPET_OK;
+    }
   }
   const int ntiles = npad / kTile;
   FieldOut o;
@@ -1013,8 +1013,10 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   int K = ctx->tune[4][0] > 0 ? ctx->tune[4][0] : 2;  // as the single-frame grid kernel
   std::vector<int32_t> geo(4 * (size_t)F), ax_off(F), blk;
   std::vector<int64_t> out_off(F);
-  std::vector<FarGrid> fars;  // frames of the interpolating path, as field_launch chooses
-  std::vector<int> smalls;    // frames of the FP64 pair terms (smallfield.hip)
+  // frames of the interpolating path (fargrid.hip) and of the FP64 pair terms
+  // (smallfield.hip); the others stay direct
+  std::vector<FarGrid> grids;
+  std::vector<int> fars, smalls, direct;
   long long small_pts = 0;
   const bool may_far = mode == kModeAuto && !(flags & CPET_F_OUT_F64) && ctx->tune[4][0] <= 0;
   const int ch_total = chg_off.empty() ? 0 : chg_off.back();
@@ -1037,9 +1039,10 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
     pts += (long long)nx * ny * nz;
     const int npad = chg_off[f + 1] - chg_off[f];
     if (may_far && far_grid_ok(nx, ny, nz, npad, kFarMinPairsBatch)) {
-      fars.push_back(FarGrid{{nx, ny, nz},
-                             {ax_off[f], ax_off[f] + nx, ax_off[f] + nx + ny},
-                             npad, chg_off[f], out_off[f]});
+      grids.push_back(FarGrid{{nx, ny, nz},
+                              {ax_off[f], ax_off[f] + nx, ax_off[f] + nx + ny},
+                              npad, chg_off[f], out_off[f]});
+      fars.push_back(f);
       continue;
     }
     const long long M = (long long)nx * ny * nz;
@@ -1048,7 +1051,13 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
       small_pts += M;
       continue;
     }
-    const long long lanes = (long long)nx * ny * nzc;
+    direct.push_back(f);
+  }
+  std::shared_ptr<const FarPlan> plan;
+  if (!fars.empty() && !(plan = far_grid_plan(ctx, grids, E_out != nullptr, phi_out != nullptr)))
+    direct.insert(direct.end(), fars.begin(), fars.end());
+  for (int f : direct) {
+    const long long lanes = (long long)geo[4 * f] * geo[4 * f + 1] * geo[4 * f + 3];
     for (long long b = 0; b < (lanes + 255) / 256; ++b) {
       blk.push_back(f);
       blk.push_back((int32_t)b);
@@ -1067,11 +1076,9 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   ctx->all_f64 = E_out ? small_pts : 0;
   int rc = prof_mark(ctx, 0);
   if (rc) return rc;
-  if (!fars.empty()) {
+  if (plan) {
     const float* const axes[3] = {axes_dev, axes_dev, axes_dev};
-    if ((rc = far_grid_launch(ctx, fars, axes, ch, E_out != nullptr, phi_out != nullptr,
-                              soften != 0, E_out, phi_out)))
-      return rc;
+    if ((rc = far_grid_run(ctx, *plan, axes, ch, soften != 0, E_out, phi_out))) return rc;
   }
   if (blk.empty()) {  // every frame took it
     for (int i = 1; i < 3; ++i)

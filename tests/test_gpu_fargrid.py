@@ -320,3 +320,41 @@ def test_captured_batch_of_several_scratch_groups(gpu_ctx):
         b = want[k * M:(k + 1) * M]
         scale = float(one.double().square().mean().sqrt())
         assert float((one - b).abs().max()) <= 1e-7 * scale + 5e-6 * float(one.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, charges", [((217, 217, 217), 200), ((217, 218, 217), 45000)])
+def test_largest_plan(oracle_mod, n, charges):
+    """Four halvings on every axis (4,681 cells, 80 KB of LDS in the classification), with few
+    charges, and with so many that the near lists of all leaves would need 740 MB: right, and
+    within 1 GiB of scratch (and the quarter that the context adds)."""
+    import torch
+
+    from pycpet_amd import _native as nat, batch, ops
+
+    rng = np.random.default_rng(charges)
+    x = rng.uniform(-25, 25, (charges, 3)).astype(np.float32)
+    q = rng.normal(0, 0.4, charges).astype(np.float32)
+    x[:40] *= np.float32(0.15)  # in the box
+    axes = [np.linspace(-5.4, 5.4, k).astype(np.float32) for k in n]
+    T = lambda a: torch.from_numpy(a).cuda()
+    xd, qd, ad = T(x), T(q), [T(a) for a in axes]
+    out = torch.empty((int(np.prod(n)), 3), device="cuda")  # what the call's result will use
+    del out
+    ctx = nat.Context(0)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    E, _ = ops.field_grid(*ad, xd, qd, ctx=ctx)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 1.3 * 2**30
+    _check(axes, x, q, E.cpu().numpy(), None, oracle_mod)
+    few = {"x": xd[:9000], "q": qd[:9000], "axes": [a[::5].contiguous() for a in ad]}
+    big = {"x": xd, "q": qd, "axes": ad}
+    out = batch.batch_volume([few, big, few], ctx=ctx)  # in a batch: a launch of its own
+    scale = float(E.double().square().mean().sqrt())
+    assert float((out[1][0] - E).abs().max()) <= 1e-7 * scale + 5e-6 * float(E.abs().max())
+    for k in (0, 2):
+        _check([a[::5] for a in axes], x[:9000], q[:9000], out[k][0].cpu().numpy(), None,
+               oracle_mod)
+    del E, out
+    ctx.close()
