@@ -401,12 +401,22 @@ int cpet_order_stats(cpet_ctx *ctx, int64_t n, int cols, const double *x, int n_
                      const int32_t *sel_cols, const int64_t *sel_ranks, double *values,
                      int64_t *nan_counts, uint32_t flags);
 
-/* Copies n host arrays, src[i] of bytes[i] bytes, one behind the other to the
- * device memory at dst, on the context's stream.  The arrays may be reused
- * when a later call on the context has waited for the stream.  No counterpart
- * in the reference. */
-int cpet_upload_rows(cpet_ctx *ctx, int n, const void *const *src, const int64_t *bytes,
-                     void *dst);
+/* The same two of host rows that lie frame by frame: feats[f] / x[f] holds the
+ * rows offsets[f] .. offsets[f+1]-1 (NULL for a frame without rows; offsets
+ * as above), copied behind one another to the context's buffer.  The rows
+ * stay there: *held, 0 before the first call on these arrays, is set to the
+ * number under which they do, and another call with that number and the same,
+ * unchanged arrays does not copy them again, unless a call in between (of any
+ * thread) has put something else there.  Host results; each call waits for
+ * its work.  CPET_F_COUNTS is the only flag.  No counterpart in the
+ * reference. */
+int cpet_cluster_histograms_rows(cpet_ctx *ctx, int F, const int64_t *offsets,
+                                 const double *const *feats, int nb_d, const double *edges_d,
+                                 int nb_c, const double *edges_c, double *hists, uint64_t *held,
+                                 uint32_t flags);
+int cpet_order_stats_rows(cpet_ctx *ctx, int F, const int64_t *offsets, const double *const *x,
+                          int cols, int n_sel, const int32_t *sel_cols, const int64_t *sel_ranks,
+                          double *values, int64_t *nan_counts, uint64_t *held);
 
 /* out (F,F) double: out[i][j] = sum over bins with h_i + h_j != 0 of
  * (h_i - h_j)^2 / (h_i + h_j), halved; zero diagonal.  Replaces

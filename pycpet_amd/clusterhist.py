@@ -13,9 +13,9 @@ frame's features, bin width 2 * IQR / n^(1/3) (scipy.stats.iqr, n the row
 count, or its mean when frames differ in length), int((max - min) / width)
 bins, and the edges numpy.histogram2d builds from (bins, range).  The min,
 max and the two quartiles come from exact order statistics selected on the
-GPU (cpet_order_stats), combined on the host with numpy.percentile's linear
+GPU (cpet_order_stats_rows), combined on the host with numpy.percentile's linear
 interpolation step for step.  The .top files are read by cpet_read_rows; the
-histograms (cpet_cluster_histograms) and the distance matrix
+histograms (cpet_cluster_histograms_rows) and the distance matrix
 (cpet_chi2_matrix) run on the GPU.
 """
 from __future__ import annotations
@@ -86,35 +86,29 @@ def _binning_count(features):
     return lens[0]
 
 
-def _rows(features):
-    """The frames as contiguous (L_f, 2) float64 arrays and their row offsets."""
-    feats = [np.ascontiguousarray(np.asarray(f, np.float64).reshape(-1, 2)) for f in features]
-    off = np.zeros(len(feats) + 1, np.int64)
-    off[1:] = np.cumsum([len(f) for f in feats])
-    return feats, off
-
-
-def _upload(feats, off, ctx):
-    """All rows in order as one (P, 2) device tensor, each frame copied from
-    where it lies: the order statistics and the histograms both read it.
+class _Rows:
+    """The frames' contiguous (L_f, 2) float64 rows and their offsets, as the
+    library takes them: copied to the device frame by frame from where they
+    lie, and kept there (`held`) from the order statistics to the histograms.
     Joining the frames on the host and sending the result to each of the two
-    took 9.9 ms of a 14.7 ms step (256 frames of 20,000 rows), this 3.7."""
-    import torch
+    took 9.9 ms of a 14.7 ms step (256 frames of 20,000 rows), this 3.7.  Both
+    calls are complete in themselves, so threads may share the context: rows
+    that another call has replaced are copied again."""
 
-    dev = torch.device("cuda", ctx.device)
-    ctx.set_stream(torch.cuda.current_stream(dev).cuda_stream)
-    rows = torch.empty((max(1, int(off[-1])), 2), dtype=torch.float64, device=dev)
-    src = (ctypes.c_void_p * len(feats))(*(f.ctypes.data for f in feats))
-    sizes = np.array([f.nbytes for f in feats], np.int64)
-    nat.check(ctx.lib.cpet_upload_rows(ctx.handle, len(feats), src, sizes.ctypes.data,
-                                       rows.data_ptr()), ctx.lib)
-    return rows
+    def __init__(self, features):
+        self.feats = [np.ascontiguousarray(np.asarray(f, np.float64).reshape(-1, 2))
+                      for f in features]
+        self.off = np.zeros(len(self.feats) + 1, np.int64)
+        self.off[1:] = np.cumsum([len(f) for f in self.feats])
+        self.count = int(self.off[-1])
+        self.ptrs = (ctypes.c_void_p * len(self.feats))(*(f.ctypes.data for f in self.feats))
+        self.held = ctypes.c_uint64(0)
 
 
 def _flatten(features):
-    feats, off = _rows(features)
-    allf = np.concatenate(feats) if off[-1] else np.zeros((0, 2))
-    return feats, off, allf
+    rows = _Rows(features)
+    allf = np.concatenate(rows.feats) if rows.count else np.zeros((0, 2))
+    return rows.feats, rows.off, allf
 
 
 def _lerp_points(count, q):
@@ -158,19 +152,20 @@ def _order_stat_ranks(count):
     return sorted(ranks)
 
 
-def _column_stats(rows, P, ctx):
-    """[(min, max, iqr)] of the two feature columns of the P device rows, from
-    order statistics selected on the GPU (cpet_order_stats: exact elements of
-    the column)."""
+def _column_stats(rows, ctx):
+    """[(min, max, iqr)] of the two feature columns, from order statistics
+    selected on the GPU (cpet_order_stats_rows: exact elements of the column)."""
+    P = rows.count
     ranks = _order_stat_ranks(P)
     plan = [(c, r) for c in range(2) for r in ranks]
     cols = np.array([c for c, _ in plan], np.int32)
     rk = np.array([r for _, r in plan], np.int64)
     vals = np.empty(len(plan), np.float64)
     nans = np.zeros(2, np.int64)
-    nat.check(ctx.lib.cpet_order_stats(ctx.handle, P, 2, rows.data_ptr(), len(plan),
-                                       cols.ctypes.data, rk.ctypes.data, vals.ctypes.data,
-                                       nans.ctypes.data, nat.F_DEVICE), ctx.lib)
+    nat.check(ctx.lib.cpet_order_stats_rows(
+        ctx.handle, len(rows.feats), rows.off.ctypes.data, rows.ptrs, 2, len(plan),
+        cols.ctypes.data, rk.ctypes.data, vals.ctypes.data, nans.ctypes.data,
+        ctypes.byref(rows.held)), ctx.lib)
     at = {key: k for k, key in enumerate(plan)}
     return [_stats_from_order(P, lambda r, c=c: vals[at[(c, r)]], int(nans[c]))
             for c in range(2)]
@@ -195,10 +190,10 @@ def _edges_from_stats(stats, n):
     return ed, ec
 
 
-def _edges(rows, P, n, ctx):
-    if P == 0:
+def _edges(rows, n, ctx):
+    if rows.count == 0:
         np.max(np.zeros((0, 2))[:, 0])  # numpy's error for an empty reduction, as the reference
-    return _edges_from_stats(_column_stats(rows, P, ctx), n)
+    return _edges_from_stats(_column_stats(rows, ctx), n)
 
 
 def histogram_edges(features: Sequence[np.ndarray],
@@ -206,8 +201,7 @@ def histogram_edges(features: Sequence[np.ndarray],
     """The shared (distance, curvature) bin edges of make_histograms."""
     ctx = ctx or nat.default_context()
     n = _binning_count(features)
-    feats, off = _rows(features)
-    return _edges(_upload(feats, off, ctx), int(off[-1]), n, ctx)
+    return _edges(_Rows(features), n, ctx)
 
 
 def histograms_from_features(features: Sequence[np.ndarray], edges=None,
@@ -215,31 +209,27 @@ def histograms_from_features(features: Sequence[np.ndarray], edges=None,
     """(F, nd*nc) normalised histograms of per-frame (L_f, 2) features."""
     ctx = ctx or nat.default_context()
     n = _binning_count(features) if edges is None else None
-    feats, off = _rows(features)
-    rows = _upload(feats, off, ctx)
-    ed, ec = edges if edges is not None else _edges(rows, int(off[-1]), n, ctx)
-    return _histograms(off, rows, ed, ec, ctx, 0)
+    rows = _Rows(features)
+    ed, ec = edges if edges is not None else _edges(rows, n, ctx)
+    return _histograms(rows, ed, ec, ctx, 0)
 
 
-def _histograms(off, rows, ed, ec, ctx, flags) -> np.ndarray:
-    """(F, nd*nc) histograms of the device rows over the shared edges."""
-    import torch
-
+def _histograms(rows, ed, ec, ctx, flags) -> np.ndarray:
+    """(F, nd*nc) histograms of the rows over the shared edges."""
     ed = np.ascontiguousarray(ed, np.float64)
     ec = np.ascontiguousarray(ec, np.float64)
     nd, nc = len(ed) - 1, len(ec) - 1
-    out = torch.empty((len(off) - 1, max(0, nd * nc)), dtype=torch.float64, device=rows.device)
-    nat.check(ctx.lib.cpet_cluster_histograms(
-        ctx.handle, len(off) - 1, off.ctypes.data, rows.data_ptr(), nd, ed.ctypes.data, nc,
-        ec.ctypes.data, out.data_ptr(), flags | nat.F_DEVICE | nat.F_NO_SYNC), ctx.lib)
-    return out.cpu().numpy()
+    out = np.empty((len(rows.feats), max(0, nd * nc)), np.float64)
+    nat.check(ctx.lib.cpet_cluster_histograms_rows(
+        ctx.handle, len(rows.feats), rows.off.ctypes.data, rows.ptrs, nd, ed.ctypes.data, nc,
+        ec.ctypes.data, out.ctypes.data, ctypes.byref(rows.held), flags), ctx.lib)
+    return out
 
 
-def _histogram_counts(off, rows, ed, ec, ctx) -> np.ndarray:
-    """(F, nd, nc) float64 bin counts over the shared edges (cpet_cluster_histograms
-    with CPET_F_COUNTS)."""
-    out = _histograms(off, rows, ed, ec, ctx, nat.F_COUNTS)
-    return out.reshape(len(off) - 1, len(ed) - 1, len(ec) - 1)
+def _histogram_counts(rows, ed, ec, ctx) -> np.ndarray:
+    """(F, nd, nc) float64 bin counts over the shared edges (CPET_F_COUNTS)."""
+    out = _histograms(rows, ed, ec, ctx, nat.F_COUNTS)
+    return out.reshape(len(rows.feats), len(ed) - 1, len(ec) - 1)
 
 
 def _read_topo_any_sep(path) -> np.ndarray:
@@ -299,10 +289,9 @@ def make_histograms_mem(topo_files, output_dir, plot=False,
         n = np.mean(lens)
     else:
         n = lens[0]
-    feats, off = _rows(feats)
-    rows = _upload(feats, off, ctx)
-    ed, ec = _edges(rows, int(off[-1]), n, ctx)
-    counts = _histogram_counts(off, rows, ed, ec, ctx)
+    rows = _Rows(feats)
+    ed, ec = _edges(rows, n, ctx)
+    counts = _histogram_counts(rows, ed, ec, ctx)
     hist_list = []
     for f, c in zip(topo_files, counts):
         outfile = os.path.join(output_dir, f"{str(f).split('/')[-1][:-4]}_hist.npy")

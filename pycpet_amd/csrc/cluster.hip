@@ -238,17 +238,72 @@ __global__ void select_pick_kernel(int T, SelTarget* __restrict__ tg, int pass,
   if (pass == kSelPasses - 1) values[t] = key_value(pre);
 }
 
+// Where a call's rows come from: one array (on the device, or copied to it), or
+// one host array per frame, copied behind one another.  The rows of the latter stay
+// in the context's buffer, under a number, until a call puts something else there.
+struct Rows {
+  const double* one = nullptr;
+  bool dev = false;
+  int F = 0;                          // frames, else 0
+  const int64_t* offsets = nullptr;   // (F+1) first row of each
+  const double* const* frames = nullptr;
+  uint64_t* held = nullptr;
+};
+
+int check_rows(const char* who, const Rows& r) {
+  if (r.F < 0 || (r.F == 0) != (r.frames == nullptr) || (r.F && (!r.offsets || !r.held))) {
+    set_error("%s: bad arguments", who);
+    return CPET_ERR_ARG;
+  }
+  for (int f = 0; f < r.F; ++f)
+    if (r.offsets[0] != 0 || r.offsets[f] > r.offsets[f + 1] ||
+        (r.offsets[f] < r.offsets[f + 1] && !r.frames[f])) {
+      set_error("%s: offsets must start at 0 and not decrease, and frame %d's rows exist", who, f);
+      return CPET_ERR_ARG;
+    }
+  return CPET_OK;
+}
+
+// The `bytes` of all rows on the device.  Called with the context locked.
+int stage_rows(cpet_ctx* ctx, const Rows& r, size_t bytes, int cols, const void** out) {
+  if (!r.F) {
+    if (!r.dev) ctx->rows_held = 0;
+    return stage_in(ctx, kSlotCluster0, r.one, bytes, r.dev, out);
+  }
+  void* d = nullptr;
+  if (*r.held && *r.held == ctx->rows_held && bytes == ctx->rows_bytes) {
+    *out = ctx->bufs[kSlotCluster0].ptr;
+    return CPET_OK;
+  }
+  ctx->rows_held = 0;
+  const int rc = ctx_buf(ctx, kSlotCluster0, bytes, &d);
+  if (rc) return rc;
+  for (int f = 0; f < r.F; ++f) {
+    const size_t first = (size_t)r.offsets[f] * cols, n = (size_t)r.offsets[f + 1] * cols - first;
+    if (n)
+      CPET_HIP_TRY(hipMemcpyAsync((double*)d + first, r.frames[f], n * sizeof(double),
+                                  hipMemcpyHostToDevice, ctx->stream));
+  }
+  *out = d;
+  return CPET_OK;
+}
+
+// Numbers the rows of a call that has waited for its copies.
+void hold_rows(cpet_ctx* ctx, const Rows& r, size_t bytes) {
+  if (!r.F || (ctx->rows_held && *r.held == ctx->rows_held)) return;
+  ctx->rows_bytes = bytes;
+  *r.held = ctx->rows_held = ++ctx->rows_last;
+}
+
 }  // namespace
 }  // namespace cpet
 
 using namespace cpet;
 
-extern "C" {
-
-int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const double* feats,
-                            int nb_d, const double* edges_d, int nb_c, const double* edges_c,
-                            double* hists, uint32_t flags) {
-  if (!ctx || F <= 0 || !offsets || !feats || nb_d <= 0 || nb_c <= 0 || !edges_d ||
+static int histograms(cpet_ctx* ctx, const Rows& rows, int F, const int64_t* offsets, int nb_d,
+                      const double* edges_d, int nb_c, const double* edges_c, double* hists,
+                      uint32_t flags) {
+  if (!ctx || F <= 0 || !offsets || (!rows.F && !rows.one) || nb_d <= 0 || nb_c <= 0 || !edges_d ||
       !edges_c || !hists) {
     set_error("cpet_cluster_histograms: bad arguments");
     return CPET_ERR_ARG;
@@ -270,6 +325,8 @@ int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const 
       set_error("cpet_cluster_histograms: curvature edges must increase");
       return CPET_ERR_ARG;
     }
+  int rc = check_rows("cpet_cluster_histograms_rows", rows);
+  if (rc) return rc;
   const long long P = offsets[F];
   const long long B = (long long)nb_d * nb_c;
   if (B > (1LL << 28)) {
@@ -277,12 +334,12 @@ int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const 
     return CPET_ERR_ARG;
   }
   std::lock_guard<std::mutex> lk(ctx->mu);
-  int rc = ctx_activate(ctx);
+  rc = ctx_activate(ctx);
   if (rc) return rc;
   hipStream_t st = ctx->stream;
   const void* dfeats = nullptr;
-  if (P > 0 && (rc = stage_in(ctx, kSlotCluster0, feats, (size_t)P * 2 * sizeof(double), dev, &dfeats)))
-    return rc;
+  const size_t row_bytes = (size_t)P * 2 * sizeof(double);
+  if (P > 0 && (rc = stage_rows(ctx, rows, row_bytes, 2, &dfeats))) return rc;
   // small tables: offsets, edges, counts in one buffer
   const size_t o_off = 0;
   const size_t o_ed = round_up((int)((F + 1) * sizeof(long long)), 256);
@@ -313,36 +370,14 @@ int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const 
   CPET_HIP_TRY(hipGetLastError());
   if (!dev) CPET_HIP_TRY(hipMemcpyAsync(hists, dh, (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, st));
   if (!dev || !(flags & CPET_F_NO_SYNC)) CPET_HIP_TRY(hipStreamSynchronize(st));
+  if (P > 0) hold_rows(ctx, rows, row_bytes);
   return CPET_OK;
 }
 
-int cpet_upload_rows(cpet_ctx* ctx, int n, const void* const* src, const int64_t* bytes,
-                     void* dst) {
-  if (!ctx || n < 0 || (n > 0 && (!src || !bytes || !dst))) {
-    set_error("cpet_upload_rows: bad arguments");
-    return CPET_ERR_ARG;
-  }
-  for (int i = 0; i < n; ++i)
-    if (bytes[i] < 0 || (bytes[i] > 0 && !src[i])) {
-      set_error("cpet_upload_rows: array %d is NULL or of negative size", i);
-      return CPET_ERR_ARG;
-    }
-  std::lock_guard<std::mutex> lk(ctx->mu);
-  const int rc = ctx_activate(ctx);
-  if (rc) return rc;
-  char* to = (char*)dst;
-  for (int i = 0; i < n; ++i) {
-    if (bytes[i])
-      CPET_HIP_TRY(hipMemcpyAsync(to, src[i], (size_t)bytes[i], hipMemcpyHostToDevice, ctx->stream));
-    to += bytes[i];
-  }
-  return CPET_OK;
-}
-
-int cpet_order_stats(cpet_ctx* ctx, int64_t n, int cols, const double* x, int n_sel,
-                     const int32_t* sel_cols, const int64_t* sel_ranks, double* values,
-                     int64_t* nan_counts, uint32_t flags) {
-  if (!ctx || n <= 0 || cols <= 0 || cols > kSelMaxCols || !x || n_sel <= 0 ||
+static int order_stats(cpet_ctx* ctx, const Rows& rows, int64_t n, int cols, int n_sel,
+                       const int32_t* sel_cols, const int64_t* sel_ranks, double* values,
+                       int64_t* nan_counts) {
+  if (!ctx || n <= 0 || cols <= 0 || cols > kSelMaxCols || (!rows.F && !rows.one) || n_sel <= 0 ||
       n_sel > kSelMaxTargets || !sel_cols || !sel_ranks || !values) {
     set_error("cpet_order_stats: bad arguments (1 <= cols <= %d, 1 <= n_sel <= %d)",
               kSelMaxCols, kSelMaxTargets);
@@ -362,14 +397,13 @@ int cpet_order_stats(cpet_ctx* ctx, int64_t n, int cols, const double* x, int n_
     }
     tgh[k] = SelTarget{0ull, (unsigned long long)sel_ranks[k], (int)sel_cols[k], 0};
   }
-  const bool dev = (flags & CPET_F_DEVICE) != 0;
   std::lock_guard<std::mutex> lk(ctx->mu);
   int rc = ctx_activate(ctx);
   if (rc) return rc;
   hipStream_t st = ctx->stream;
   const long long total = (long long)n * cols;
   const void* dx = nullptr;
-  if ((rc = stage_in(ctx, kSlotCluster0, x, (size_t)total * sizeof(double), dev, &dx))) return rc;
+  if ((rc = stage_rows(ctx, rows, (size_t)total * sizeof(double), cols, &dx))) return rc;
   // tables: targets | per-pass digit counts | NaN counts | values
   const size_t o_tg = 0;
   const size_t o_h = 512;
@@ -404,9 +438,57 @@ int cpet_order_stats(cpet_ctx* ctx, int64_t n, int cols, const double* x, int n_
   CPET_HIP_TRY(hipMemcpyAsync(values, dval, n_sel * sizeof(double), hipMemcpyDeviceToHost, st));
   CPET_HIP_TRY(hipMemcpyAsync(nanh, dnan, cols * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
   CPET_HIP_TRY(hipStreamSynchronize(st));
+  hold_rows(ctx, rows, (size_t)total * sizeof(double));
   if (nan_counts)
     for (int c = 0; c < cols; ++c) nan_counts[c] = (int64_t)nanh[c];
   return CPET_OK;
+}
+
+extern "C" {
+
+int cpet_cluster_histograms(cpet_ctx* ctx, int F, const int64_t* offsets, const double* feats,
+                            int nb_d, const double* edges_d, int nb_c, const double* edges_c,
+                            double* hists, uint32_t flags) {
+  Rows rows;
+  rows.one = feats;
+  rows.dev = (flags & CPET_F_DEVICE) != 0;
+  return histograms(ctx, rows, F, offsets, nb_d, edges_d, nb_c, edges_c, hists, flags);
+}
+
+int cpet_cluster_histograms_rows(cpet_ctx* ctx, int F, const int64_t* offsets,
+                                 const double* const* feats, int nb_d, const double* edges_d,
+                                 int nb_c, const double* edges_c, double* hists, uint64_t* held,
+                                 uint32_t flags) {
+  Rows rows;
+  rows.F = F;
+  rows.offsets = offsets;
+  rows.frames = feats;
+  rows.held = held;
+  return histograms(ctx, rows, F, offsets, nb_d, edges_d, nb_c, edges_c, hists,
+                    flags & CPET_F_COUNTS);
+}
+
+int cpet_order_stats(cpet_ctx* ctx, int64_t n, int cols, const double* x, int n_sel,
+                     const int32_t* sel_cols, const int64_t* sel_ranks, double* values,
+                     int64_t* nan_counts, uint32_t flags) {
+  Rows rows;
+  rows.one = x;
+  rows.dev = (flags & CPET_F_DEVICE) != 0;
+  return order_stats(ctx, rows, n, cols, n_sel, sel_cols, sel_ranks, values, nan_counts);
+}
+
+int cpet_order_stats_rows(cpet_ctx* ctx, int F, const int64_t* offsets, const double* const* x,
+                          int cols, int n_sel, const int32_t* sel_cols, const int64_t* sel_ranks,
+                          double* values, int64_t* nan_counts, uint64_t* held) {
+  Rows rows;
+  rows.F = F;
+  rows.offsets = offsets;
+  rows.frames = x;
+  rows.held = held;
+  const int rc = check_rows("cpet_order_stats_rows", rows);
+  if (rc) return rc;
+  return order_stats(ctx, rows, offsets ? offsets[F] : 0, cols, n_sel, sel_cols, sel_ranks, values,
+                     nan_counts);
 }
 
 int cpet_chi2_matrix(cpet_ctx* ctx, int F, int B, const double* hists, double* out,
@@ -421,8 +503,10 @@ int cpet_chi2_matrix(cpet_ctx* ctx, int F, int B, const double* hists, double* o
   if (rc) return rc;
   hipStream_t st = ctx->stream;
   const void* dh = nullptr;
-  if ((rc = stage_in(ctx, kSlotCluster0, hists, (size_t)F * B * sizeof(double), dev, &dh)))
-    return rc;
+  Rows in;
+  in.one = hists;
+  in.dev = dev;
+  if ((rc = stage_rows(ctx, in, (size_t)F * B * sizeof(double), 1, &dh))) return rc;
   double* dout = out;
   if (!dev) {
     void* ob = nullptr;

@@ -94,6 +94,9 @@ struct cpet_ctx {
   // device counter of the points the last auto-mode field call recomputed
   // in FP64 (null when that call had no check)
   int* fix_count = nullptr;
+  // rows that the cluster step's buffer holds (0: none): see stage_rows
+  uint64_t rows_held = 0, rows_last = 0;
+  size_t rows_bytes = 0;
   long long all_f64 = 0;  // the points of a call that computed every one in FP64
   // last host table uploaded per key (upload_table): an identical table at
   // the same device address is not copied again, so repeated calls of one

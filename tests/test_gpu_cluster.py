@@ -279,3 +279,81 @@ def test_rows_uploaded_frame_by_frame(gpu_ctx):
             np.testing.assert_array_equal(h, want / want.sum())
         else:
             assert np.isnan(h).all()
+
+
+def _feature_frames(seed, F=9, rows=400):
+    rng = np.random.default_rng(seed)
+    return [np.abs(rng.normal(1.0 + 0.3 * seed, 0.4, (rows, 2))) for _ in range(F)]
+
+
+def test_context_stays_as_it_was(gpu_ctx):
+    """The cluster step runs on the stream that the context has, and leaves it."""
+    import torch
+
+    from pycpet_amd import clusterhist as CH
+
+    ctx = gpu_ctx
+    own = torch.cuda.Stream()
+    before = ctx.stream()
+    try:
+        ctx.set_stream(own.cuda_stream)
+        CH.histograms_from_features(_feature_frames(1), ctx=ctx)
+        assert ctx.stream() == own.cuda_stream
+        CH.histogram_edges(_feature_frames(1), ctx=ctx)
+        assert ctx.stream() == own.cuda_stream
+    finally:
+        torch.cuda.synchronize()
+        ctx.set_stream(before)
+
+
+def test_threads_share_a_context(gpu_ctx):
+    """Cluster steps of several threads on one context, each under its own torch stream, and
+    another step between a step's order statistics and its histograms: every result is the one
+    of the same step run alone."""
+    import threading
+
+    import torch
+
+    from pycpet_amd import clusterhist as CH
+
+    sets = [_feature_frames(k, F=5 + k, rows=300 + 517 * k) for k in range(4)]
+    want = [CH.histograms_from_features(s, ctx=gpu_ctx) for s in sets]
+    edges_of, nested = CH._edges_from_stats, []
+
+    def between(stats, n):
+        if not nested:
+            nested.append(None)
+            nested[0] = CH.histograms_from_features(sets[1], ctx=gpu_ctx)
+        return edges_of(stats, n)
+
+    CH._edges_from_stats = between
+    try:
+        np.testing.assert_array_equal(CH.histograms_from_features(sets[2], ctx=gpu_ctx), want[2])
+        np.testing.assert_array_equal(nested[0], want[1])
+    finally:
+        CH._edges_from_stats = edges_of
+    wrong = []
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                if not np.array_equal(CH.histograms_from_features(sets[k], ctx=gpu_ctx), want[k]):
+                    wrong.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+def test_cluster_step_without_torch(gpu_ctx, monkeypatch):
+    """The step needs numpy and the library only."""
+    import sys
+
+    from pycpet_amd import clusterhist as CH
+
+    monkeypatch.setitem(sys.modules, "torch", None)
+    hist = CH.histograms_from_features(_feature_frames(2), ctx=gpu_ctx)
+    np.testing.assert_allclose(hist.sum(1), 1.0)
