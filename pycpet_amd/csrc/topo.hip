@@ -1796,8 +1796,10 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
   // 2. propagate
   int G = ctx->tune[2][1];
   // with the chunk-lane form a workgroup need not have 64 streamlines: every
-  // CU gets a share
-  const int gmax = d_chunks ? L : (L + 63) / 64;
+  // CU gets a share, and no more than one (its LDS): another one's streamlines,
+  // which it has before it starts, would wait for the first one's last, and
+  // places and counter stay below 2^31
+  const int gmax = d_chunks ? std::min(L, ctx->num_cus) : (L + 63) / 64;
   // One 16-wave workgroup per CU: the fewest slots that keep every SIMD fed
   // (4 waves each, with the charge loads prefetched), so the tail of long
   // streamlines still running after the queue drains is shortest.

@@ -87,3 +87,28 @@ def test_chunk_lanes_of_a_batch(gpu_ctx):
                                ctx=gpu_ctx))
     finally:
         gpu_ctx.set_tuning(2, 0, 0)
+
+
+@pytest.mark.gpu
+def test_asked_for_workgroups_are_bounded(gpu_ctx):
+    """More workgroups asked for than fit the chip, on so many streamlines that 64 places for
+    each would pass 2^31: the results of the library's own choice."""
+    import torch
+
+    from pycpet_amd import ops
+
+    L = 2**31 // 63 + 1000
+    g = torch.Generator("cuda").manual_seed(1)
+    rng = np.random.default_rng(1)
+    starts = torch.rand((L, 3), device="cuda", generator=g).sub_(0.5)
+    n_iter = torch.ones(L, dtype=torch.int32, device="cuda")
+    x = torch.from_numpy((rng.standard_normal((200, 3)) * 9).astype(np.float32)).cuda()
+    q = torch.from_numpy(rng.normal(0, 0.4, 200).astype(np.float32)).cuda()
+    args = (starts, n_iter, 0.01, np.ones(3, np.float32), x, q)
+    want = ops.topo(*args, ctx=gpu_ctx).feats
+    gpu_ctx.set_tuning(2, 16, L)
+    try:
+        got = ops.topo(*args, ctx=gpu_ctx).feats
+    finally:
+        gpu_ctx.set_tuning(2, 0, 0)
+    assert torch.equal(got.view(torch.int64), want.view(torch.int64))
