@@ -1230,10 +1230,15 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
   }
 }
 
-// A slot's first place in the queue: the places go round the workgroups, so
-// that each has a like share of the long streamlines.  A slot that is not used
-// gets one past the end.
+// A slot's first place in the queue.  In the chunk-lane form the places go round
+// the workgroups, so that each has a like share of the long streamlines, and a
+// slot that is not used gets one past the end.  In the slice form, where an
+// evaluation costs the same however few slots are in use, a workgroup takes
+// neighbours of the longest-first order, so that those with short streamlines are
+// done soon: 2,000 charges, 20,000 streamlines with 8-wave workgroups 27.7 ms, 39.8
+// with the places going round; 16 charges, 400,000 in one-wave workgroups 6.0 and 8.2.
 __device__ __forceinline__ int first_place(const PropArgs& a, int lane) {
+  if (!a.chunks) return (int)blockIdx.x * 64 + lane;
   return lane < a.slots ? lane * (int)gridDim.x + (int)blockIdx.x : a.L;
 }
 
@@ -1767,7 +1772,7 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
   const bool f64 = src == kSrcChargeF64 || src == kSrcChargeF64Rk4;
   const int rps = src == kSrcDipoleRef || src == kSrcDipolePhys ? 2 : 1;
   float4* d_chunks = nullptr;
-  if (S == kSplitSlices && !f64) {
+  if (S == kSplitSlices && !f64 && !d_far) {  // the far form has no use for fewer slots
     const int groups = chunk_groups(npad);
     d_chunks = (float4*)ctx_buf_try(ctx, kSlotChunks,
                                     (size_t)groups * kChunkQuads * 64 * rps * sizeof(float4));
@@ -1961,6 +1966,7 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   const int G0 = ctx->tune[3][1] > 0 ? ctx->tune[3][1]
                : S == 1            ? ctx->num_cus * 24
                                    : ctx->num_cus * (S >= 16 ? 1 : 2);
+  const bool want_far = S >= 4 && ctx->tune[5][0] == 2;  // the far form, for frames it is safe for
   // chunk groups of every frame (see topo_run)
   float4* d_chunks = nullptr;
   if (S == kSplitSlices) {
@@ -1981,7 +1987,7 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   // the mean: 32 -> 26 ms with 20 slots; eight frames of 10,648: 173 ms with
   // 64, 182 with 48.
   int slots = 64;
-  if (d_chunks) {
+  if (d_chunks && !want_far) {
     const int want = std::max((int)(Lt / (4LL * G0)), 64 / chunk_groups(chg_off[F] / F));
     slots = std::max(4, std::min(64, (want + 3) / 4 * 4));
   }
@@ -2081,7 +2087,7 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   // far-field records of every frame and the per-frame safety flags
   const float4* d_far = nullptr;
   const int* d_far_unsafe = nullptr;
-  if (S >= 4 && ctx->tune[5][0] == 2) {
+  if (want_far) {
     const int total = chg_off[F];
     void* fb = nullptr;
     if ((rc = ctx_buf(ctx, kSlotFar, (size_t)total * 2 * sizeof(float4) + (size_t)F * 4 + 256,
