@@ -437,13 +437,23 @@ __device__ __forceinline__ int longest_slice(int nrec, int rps) {
 // Sources of the field a streamline follows.  A policy gives the FP32
 // slice sum of the propagate kernel and the FP64 field of the epilogue.
 //
-// The 13 operations of a pair are kept together, in the order in which one
-// needs the other (a scheduling barrier after each pair).  The scheduler's own
-// order, which starts the next pairs during a pair's rsq, looks better and is
-// slower: 53.8 against 45.0 cycles a pair and wave in a loop of the pairs alone
-// (four waves per SIMD), and hand-made mixtures of two or four pairs take 46
-// to 51.  Four waves per SIMD fill a wave's waits anyway.  The one-wave walk of
-// a few sources goes without (2 % slower with it).
+// How a workgroup is compiled:
+//   kShared   up to eight waves per SIMD: workgroups of up to eight waves, and
+//             16-wave ones that share a CU or are a batch's
+//   kAlone    16 waves alone on their CU, four per SIMD
+//   kChunks   the same with the chunk-lane form beside the slice form
+enum Form : int { kShared = 0, kAlone = 1, kChunks = 2 };
+
+// With four waves per SIMD the 13 operations of a charge's pair are kept
+// together, in the order in which one needs the other (a scheduling barrier
+// after each pair).  The scheduler's own order, which starts the next pairs during
+// a pair's rsq, looks better and is slower: 53.8 against 45.0 cycles a pair and
+// wave in a loop of the pairs alone (four waves per SIMD), and hand-made mixtures
+// of two or four pairs take 46 to 51.  Four waves per SIMD fill a wave's waits
+// anyway.  With the registers for eight waves the scheduler has no room for such
+// mixtures, and the barrier costs 2 to 4 % (batches of 400 charges a frame, the
+// one-wave walk).  For dipoles it gains 2 to 3 % from some 2,000 on and costs 6 to
+// 10 % below 1,000: they have it in kChunks only (see ordered and chunk_line).
 template <bool ORDER>
 __device__ __forceinline__ void pair_order() {
   if constexpr (ORDER) __builtin_amdgcn_sched_barrier(0);
@@ -453,10 +463,11 @@ __device__ __forceinline__ void pair_order() {
 struct ChargeSrc {
   static constexpr int kRecPerSrc = 1;
   static constexpr int kComp = 3;  // the slice sums are the field components
+  __host__ __device__ static constexpr bool ordered(int form) { return form != kShared; }
   // Unsoftened field of charge records [r0, r1) at one point (the k factor
   // is applied by the caller).
   // The FP32 term of one charge at displacement d, added into f.
-  template <bool ORDER = true>
+  template <bool ORDER>
   __device__ static void pair(float dx, float dy, float dz, float q, float (&f)[3]) {
     const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
     const float ri = __builtin_amdgcn_rsqf(r2);
@@ -467,7 +478,7 @@ struct ChargeSrc {
     pair_order<ORDER>();
   }
   // The FP32 terms of one group of four charge records, added into f.
-  template <bool ORDER = true>
+  template <bool ORDER>
   __device__ static void group(float px, float py, float pz, const float4 (&c)[4],
                                float (&f)[3]) {
 #pragma unroll
@@ -483,12 +494,13 @@ struct ChargeSrc {
   }
   __device__ static void quad(const f32x4 (&d)[4], float (&f)[3]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) pair(d[0][u], d[1][u], d[2][u], d[3][u], f);
+    for (int u = 0; u < 4; ++u) pair<true>(d[0][u], d[1][u], d[2][u], d[3][u], f);
   }
+  template <bool ORDER>
   __device__ static void slice(float px, float py, float pz, const float4* __restrict__ ch,
                                int r0, int r1, double (&e)[3]) {
     stream_recs<kTile, 3>(ch, r0, r1, [&](const float4 (&c)[4], float (&f)[3]) {
-      group(px, py, pz, c, f);
+      group<ORDER>(px, py, pz, c, f);
     }, e);
   }
   // Sources [g0, g1), both multiples of 16.
@@ -527,11 +539,12 @@ template <bool PHYS>
 struct DipoleSrc {
   static constexpr int kRecPerSrc = 2;
   static constexpr int kComp = 3;
+  __host__ __device__ static constexpr bool ordered(int form) { return form == kChunks; }
   __device__ static float coef(float mx, float my, float mz, float dx, float dy, float dz) {
     return PHYS ? 3.f * fmaf(mz, dz, fmaf(my, dy, mx * dx)) : fmaf(3.f * mx, dx, fmaf(my, dy, mz * dz));
   }
   // The FP32 term of one dipole at displacement d, added into f.
-  template <bool ORDER = true>
+  template <bool ORDER>
   __device__ static void pair(float dx, float dy, float dz, float mx, float my, float mz,
                               float (&f)[3]) {
     const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
@@ -545,7 +558,7 @@ struct DipoleSrc {
     pair_order<ORDER>();
   }
   // The FP32 terms of one group of four records (two dipoles), added into f.
-  template <bool ORDER = true>
+  template <bool ORDER>
   __device__ static void group(float px, float py, float pz, const float4 (&c)[4],
                                float (&f)[3]) {
 #pragma unroll
@@ -565,12 +578,13 @@ struct DipoleSrc {
   __device__ static void quad(const f32x4 (&d)[6], float (&f)[3]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      pair(d[0][u], d[1][u], d[2][u], d[3][u], d[4][u], d[5][u], f);
+      pair<true>(d[0][u], d[1][u], d[2][u], d[3][u], d[4][u], d[5][u], f);
   }
+  template <bool ORDER>
   __device__ static void slice(float px, float py, float pz, const float4* __restrict__ ch,
                                int r0, int r1, double (&e)[3]) {
     stream_recs<2 * kTile, 3>(ch, r0, r1, [&](const float4 (&c)[4], float (&f)[3]) {
-      group(px, py, pz, c, f);
+      group<ORDER>(px, py, pz, c, f);
     }, e);
   }
   // Sources [g0, g1), both multiples of 16.
@@ -707,6 +721,8 @@ struct ChargeSrcFar {
   static constexpr int kRecPerSrc = 2;
   static constexpr int kComp = 4;   // S0, Sx, Sy, Sz
   static constexpr int kGroup = 8;  // records per scalar-load group: 4 charges
+  __host__ __device__ static constexpr bool ordered(int) { return false; }
+  template <bool ORDER>
   __device__ static void slice(float px, float py, float pz, const float4* __restrict__ ch,
                                int r0, int r1, double (&e)[4]) {
     // -2 p (exact) and |p|^2, once per evaluation
@@ -935,7 +951,7 @@ __device__ __forceinline__ void walk_slices(float px, float py, float pz, double
     if constexpr (IsF64<Src>::value)
       Src::slice64(dpx, dpy, dpz, ch, r0, r1, pv);
     else
-      Src::slice(px, py, pz, ch, r0, r1, pv);
+      Src::template slice<false>(px, py, pz, ch, r0, r1, pv);
 #pragma unroll
     for (int c = 0; c < NC; ++c) fc[c] += pv[c];
   }
@@ -989,9 +1005,9 @@ __device__ __forceinline__ void walk_groups(float px, float py, float pz,
 
 __host__ __device__ constexpr int kPartBufs(int S) { return S >= 4 ? 1 : 2; }
 
-// Whether the kernel of S waves and these sources has the chunk-lane form.
+// Whether the kernel of S waves and these sources comes in other forms than kShared.
 template <int S, class Src>
-struct HasChunks {
+struct HasForms {
   static constexpr bool value = S == kSplitSlices && HasGroup<Src>::value;
 };
 
@@ -1045,7 +1061,7 @@ __device__ __forceinline__ void split_slices(const FrameView& f, unsigned long l
   }
 }
 
-template <int S, class Src>
+template <int S, class Src, int FORM>
 __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const FrameView& f,
                                           int first_q, double* part, double* esum,
                                           int (*nsid)[64], float* cs, int lane, int wave) {
@@ -1100,9 +1116,9 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
     // the slice form takes 16 x slice pairs' time a wave, the chunk-lane form
     // that of its slot quads (of 16)
     bool split = false;
-    if constexpr (HasChunks<S, Src>::value) {
+    if constexpr (FORM == kChunks) {
       const int tiles = (__popcll(act) + 3) >> 2;
-      split = f.chunks && tiles > 0 && (15 - tiles) * f.slice >= kSplitGain;
+      split = tiles > 0 && (15 - tiles) * f.slice >= kSplitGain;
       if (split) split_slices<Src>(f, act, ex32, ey32, ez32, cs, lane, wave, fc);
     }
     if (st == kActive && !split) {
@@ -1120,7 +1136,7 @@ __device__ __forceinline__ void run_slots(const float4* __restrict__ ch, const F
         if constexpr (IsF64<Src>::value)
           Src::slice64(rk4 ? qx : px, rk4 ? qy : py, rk4 ? qz : pz, ch, f.r0, f.r1, fc);
         else
-          Src::slice(ex32, ey32, ez32, ch, f.r0, f.r1, fc);
+          Src::template slice<Src::ordered(FORM)>(ex32, ey32, ez32, ch, f.r0, f.r1, fc);
       }
     }
     const int b = NB == 1 ? 0 : par;
@@ -1246,15 +1262,14 @@ __device__ __forceinline__ int first_place(const PropArgs& a, int lane) {
 // the compiler may read charges through the scalar cache despite the
 // kernel's stores.
 //
-// The 16-wave workgroup is alone on its CU (its LDS, and one per CU is what
-// is launched), four waves per SIMD.
-template <int S, class Src>
-__global__ __launch_bounds__(64 * S, S >= 16 ? 4 : 8) void topo_propagate_kernel(
+// One 16-wave workgroup per CU is what is launched by default (kAlone, kChunks).
+template <int S, class Src, int FORM>
+__global__ __launch_bounds__(64 * S, FORM == kShared ? 8 : 4) void topo_propagate_kernel(
     const float4* __restrict__ ch, PropArgs a) {
   __shared__ double part[kPartBufs(S) * S * Src::kComp * 64];
   __shared__ double esum[Src::kComp * 64];
   __shared__ int nsid[2][64];
-  __shared__ float cs[HasChunks<S, Src>::value ? kChunkSums : 1];
+  __shared__ float cs[FORM == kChunks ? kChunkSums : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   FrameView f;
@@ -1278,7 +1293,7 @@ __global__ __launch_bounds__(64 * S, S >= 16 ? 4 : 8) void topo_propagate_kernel
   f.vgran = 4;
   f.chunks = a.chunks;
   f.slice = longest_slice(nrec, Src::kRecPerSrc);
-  run_slots<S, Src>(ch, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
+  run_slots<S, Src, FORM>(ch, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
 }
 
 // The far-field form (ChargeSrcFar) of the single-frame kernel, launched
@@ -1292,7 +1307,7 @@ __global__ __launch_bounds__(64 * S, 4) void topo_far_kernel(const float4* __res
   __shared__ double part[kPartBufs(S) * S * ChargeSrcFar::kComp * 64];
   __shared__ double esum[ChargeSrcFar::kComp * 64];
   __shared__ int nsid[2][64];
-  __shared__ float cs[HasChunks<S, ChargeSrcFar>::value ? kChunkSums : 1];
+  __shared__ float cs[1];
   if (__builtin_amdgcn_readfirstlane(*a.far_unsafe) != 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1315,7 +1330,7 @@ __global__ __launch_bounds__(64 * S, 4) void topo_far_kernel(const float4* __res
   f.vgran = gran;
   f.chunks = nullptr;
   f.slice = 0;
-  run_slots<S, ChargeSrcFar>(far, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
+  run_slots<S, ChargeSrcFar, kShared>(far, f, first_place(a, lane), part, esum, nsid, cs, lane, wave);
 }
 
 // Many frames in one persistent launch.  Workgroups claim assignments
@@ -1348,13 +1363,13 @@ struct BatchTopoArgs {
 // occupancy targets, see topo_far_kernel), each walking the whole
 // assignment list with its own counter and skipping the other form's
 // frames, so every frame runs in exactly one of them.
-template <int S, bool FAR>
+template <int S, bool FAR, int FORM>
 __device__ __forceinline__ void batch_body(const float4* __restrict__ src, BatchTopoArgs a) {
   using Src = typename std::conditional<FAR, ChargeSrcFar, ChargeSrc>::type;
   __shared__ double part[kPartBufs(S) * S * Src::kComp * 64];
   __shared__ double esum[Src::kComp * 64];
   __shared__ int nsid[2][64];
-  __shared__ float cs[HasChunks<S, Src>::value ? kChunkSums : 1];
+  __shared__ float cs[FORM == kChunks ? kChunkSums : 1];
   __shared__ int cur;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1392,7 +1407,7 @@ __device__ __forceinline__ void batch_body(const float4* __restrict__ src, Batch
       f.vgran = gran;
       f.chunks = nullptr;
       f.slice = 0;
-      run_slots<S, ChargeSrcFar>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
+      run_slots<S, ChargeSrcFar, kShared>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
     } else {
       const int nrec = __builtin_amdgcn_readfirstlane(used_records(src, c0, nc, 1, lane));
       wave_records(c0, nrec, wave, S, f.r0, f.r1);
@@ -1401,21 +1416,21 @@ __device__ __forceinline__ void batch_body(const float4* __restrict__ src, Batch
       f.vgran = 4;
       f.chunks = a.chunks ? a.chunks + (size_t)chunk_group0(c0, fr) * kChunkQuads * 64 : nullptr;
       f.slice = longest_slice(nrec, 1);
-      run_slots<S, ChargeSrc>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
+      run_slots<S, ChargeSrc, FORM>(src, f, -a.slots, part, esum, nsid, cs, lane, wave);
     }
   }
 }
 
-template <int S>
-__global__ __launch_bounds__(64 * S, S >= 16 ? 4 : 8) void topo_batch_kernel(const float4* __restrict__ ch,
-                                                            BatchTopoArgs a) {
-  batch_body<S, false>(ch, a);
+template <int S, int FORM>
+__global__ __launch_bounds__(64 * S, FORM == kShared ? 8 : 4) void topo_batch_kernel(
+    const float4* __restrict__ ch, BatchTopoArgs a) {
+  batch_body<S, false, FORM>(ch, a);
 }
 
 template <int S>
 __global__ __launch_bounds__(64 * S, 4) void topo_batch_far_kernel(
     const float4* __restrict__ far, BatchTopoArgs a) {
-  batch_body<S, true>(far, a);
+  batch_body<S, true, kShared>(far, a);
 }
 
 // ---- 3. FP64 epilogue -------------------------------------------------
@@ -1658,8 +1673,30 @@ __global__ __launch_bounds__(kEpiWaves * kEpiLanes) void topo_batch_epilogue_ker
   }
 }
 
+// Source records from which on a frame of L streamlines takes the chunk-lane form
+// (by default, one workgroup per CU).  It is compiled beside the slice form, which
+// it makes 5 to 10 % slower where slices are short (a full set of slots takes the
+// slice form in any case), and gains where slots are empty: at the end of the
+// queue, a smaller part of the call the more streamlines there are.  Slice
+// against chunk-lane form, ms, with all step limits alike (h = 0.001, cap 2,000):
+//            L = 1,000          20,000           60,000           100,000
+//   Euler    260: 4.1, 3.7      400: 5.7, 5.7    800: 18.5, 19.1  1,500: 49.4, 50.1
+//            1,000: 10.6, 6.0   800: 9.4, 9.0    1,000: 20.4, 20  5,000: 147, 147
+//            L = 2,000          20,000           60,000           150,000
+//   RK4      200: 14.7, 15.0    600: 29.6, 30.2  1,500: 125, 129  1,000: 185, 202
+//            400: 22.4, 17.0    1,000: 43, 42    2,000: 162, 161
+//   dipoles  130: 3.7, 3.9      600: 11.8, 12.2  1,000: 36.9, 38  1,000: 85.8, 92.9
+//            200: 5.1, 4.2      1,000: 18.8, 18  2,000: 74.8, 72
+// Where the limits are spread (h = 0.01, no cap) more of the call has empty slots:
+// RK4 20,000 450: 4.7, 4.2.
+long long chunk_line(int L, bool dipoles) { return std::max(300, L / (dipoles ? 25 : 64)); }
+// The same of a batch, whose frames drain one by one, for the mean of their padded
+// charges: 40 frames of 5,000 streamlines 800: 78.5, 79.8, 1,000: 82.5, 82.3 ms; 2
+// frames of 5,000 800: 9.4, 9.8, 1,000: 11.0, 10.7.
+constexpr int kBatchChunkLine = 896;
+
 template <int S, class Src>
-hipError_t launch_prop(hipStream_t st, int G, const float4* ch, const float4* far,
+hipError_t launch_prop(hipStream_t st, int G, int form, const float4* ch, const float4* far,
                        const PropArgs& a) {
   if constexpr (std::is_same<Src, ChargeSrc>::value && S >= 4) {
     if (far) {
@@ -1668,19 +1705,30 @@ hipError_t launch_prop(hipStream_t st, int G, const float4* ch, const float4* fa
       if (e != hipSuccess) return e;
     }
   }
-  hipLaunchKernelGGL((topo_propagate_kernel<S, Src>), dim3(G), dim3(64 * S), 0, st, ch, a);
+  if constexpr (HasForms<S, Src>::value) {
+    if (form != kShared) {
+      if (form == kChunks)
+        hipLaunchKernelGGL((topo_propagate_kernel<S, Src, kChunks>), dim3(G), dim3(64 * S), 0, st,
+                           ch, a);
+      else
+        hipLaunchKernelGGL((topo_propagate_kernel<S, Src, kAlone>), dim3(G), dim3(64 * S), 0, st,
+                           ch, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((topo_propagate_kernel<S, Src, kShared>), dim3(G), dim3(64 * S), 0, st, ch, a);
   return hipGetLastError();
 }
 
 template <class Src>
-hipError_t launch_prop_s(int S, hipStream_t st, int G, const float4* ch, const float4* far,
+hipError_t launch_prop_s(int S, hipStream_t st, int G, int form, const float4* ch, const float4* far,
                          const PropArgs& a) {
   switch (S) {
-    case 1: return launch_prop<1, Src>(st, G, ch, far, a);
-    case 2: return launch_prop<2, Src>(st, G, ch, far, a);
-    case 4: return launch_prop<4, Src>(st, G, ch, far, a);
-    case 8: return launch_prop<8, Src>(st, G, ch, far, a);
-    case 16: return launch_prop<16, Src>(st, G, ch, far, a);
+    case 1: return launch_prop<1, Src>(st, G, form, ch, far, a);
+    case 2: return launch_prop<2, Src>(st, G, form, ch, far, a);
+    case 4: return launch_prop<4, Src>(st, G, form, ch, far, a);
+    case 8: return launch_prop<8, Src>(st, G, form, ch, far, a);
+    case 16: return launch_prop<16, Src>(st, G, form, ch, far, a);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1772,7 +1820,15 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
   const bool f64 = src == kSrcChargeF64 || src == kSrcChargeF64Rk4;
   const int rps = src == kSrcDipoleRef || src == kSrcDipolePhys ? 2 : 1;
   float4* d_chunks = nullptr;
-  if (S == kSplitSlices && !f64 && !d_far) {  // the far form has no use for fewer slots
+  // More workgroups asked for than there are CUs, with 64 streamlines for each:
+  // two are to share a CU.
+  const int g_asked = ctx->tune[2][1];
+  const bool shared = g_asked > ctx->num_cus && L >= 64LL * g_asked;
+  int form = S == kSplitSlices && !f64 && !shared ? kAlone : kShared;
+  // one group of four charges a slice leaves nothing to order: 2.07 ms, kShared 1.98
+  if (src == kSrcCharge && N <= 4 * kSplitSlices) form = kShared;
+  // the far form has no use for fewer slots
+  if (form == kAlone && !d_far && (long long)N * rps >= chunk_line(L, rps == 2)) {
     const int groups = chunk_groups(npad);
     d_chunks = (float4*)ctx_buf_try(ctx, kSlotChunks,
                                     (size_t)groups * kChunkQuads * 64 * rps * sizeof(float4));
@@ -1784,6 +1840,7 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
         hipLaunchKernelGGL(chunk_pack_kernel<2>, dim3(4 * groups), dim3(256), 0, st, ch, 1,
                            (const int32_t*)nullptr, npad, d_chunks);
       CPET_HIP_TRY(hipGetLastError());
+      form = kChunks;
     }
   }
 
@@ -1847,12 +1904,12 @@ int topo_run(cpet_ctx* ctx, int N, int L, const float* starts,
     return CPET_ERR_ARG;
   }
   hipError_t e =
-      src == kSrcCharge         ? launch_prop_s<ChargeSrc>(S, st, G, ch, d_far, pa)
-      : src == kSrcChargeRk4    ? launch_prop_s<Rk4<ChargeSrc>>(S, st, G, ch, nullptr, pa)
-      : src == kSrcChargeF64    ? launch_prop_s<ChargeSrcF64>(S, st, G, ch, nullptr, pa)
-      : src == kSrcChargeF64Rk4 ? launch_prop_s<Rk4<ChargeSrcF64>>(S, st, G, ch, nullptr, pa)
-      : src == kSrcDipoleRef    ? launch_prop_s<DipoleSrc<false>>(S, st, G, ch, nullptr, pa)
-                                : launch_prop_s<DipoleSrc<true>>(S, st, G, ch, nullptr, pa);
+      src == kSrcCharge         ? launch_prop_s<ChargeSrc>(S, st, G, form, ch, d_far, pa)
+      : src == kSrcChargeRk4    ? launch_prop_s<Rk4<ChargeSrc>>(S, st, G, form, ch, nullptr, pa)
+      : src == kSrcChargeF64    ? launch_prop_s<ChargeSrcF64>(S, st, G, form, ch, nullptr, pa)
+      : src == kSrcChargeF64Rk4 ? launch_prop_s<Rk4<ChargeSrcF64>>(S, st, G, form, ch, nullptr, pa)
+      : src == kSrcDipoleRef    ? launch_prop_s<DipoleSrc<false>>(S, st, G, form, ch, nullptr, pa)
+                                : launch_prop_s<DipoleSrc<true>>(S, st, G, form, ch, nullptr, pa);
   if (e != hipSuccess) {
     set_error("topo propagate launch failed: %s", hipGetErrorString(e));
     return CPET_ERR_HIP;
@@ -1969,7 +2026,8 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   const bool want_far = S >= 4 && ctx->tune[5][0] == 2;  // the far form, for frames it is safe for
   // chunk groups of every frame (see topo_run)
   float4* d_chunks = nullptr;
-  if (S == kSplitSlices) {
+  const bool shared = ctx->tune[3][1] > ctx->num_cus && Lt >= 64LL * ctx->tune[3][1];
+  if (S == kSplitSlices && !shared && chg_off[F] / F >= kBatchChunkLine) {
     const int groups = chunk_group0(chg_off[F], F);
     d_chunks = (float4*)ctx_buf_try(ctx, kSlotChunks,
                                     (size_t)groups * kChunkQuads * 64 * sizeof(float4));
@@ -2132,11 +2190,16 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
     CPET_HIP_TRY(hipGetLastError());
   }
   switch (S) {
-    case 1: hipLaunchKernelGGL((topo_batch_kernel<1>), dim3(G), dim3(64), 0, st, ch, ba); break;
-    case 2: hipLaunchKernelGGL((topo_batch_kernel<2>), dim3(G), dim3(128), 0, st, ch, ba); break;
-    case 4: hipLaunchKernelGGL((topo_batch_kernel<4>), dim3(G), dim3(256), 0, st, ch, ba); break;
-    case 8: hipLaunchKernelGGL((topo_batch_kernel<8>), dim3(G), dim3(512), 0, st, ch, ba); break;
-    case 16: hipLaunchKernelGGL((topo_batch_kernel<16>), dim3(G), dim3(1024), 0, st, ch, ba); break;
+    case 1: hipLaunchKernelGGL((topo_batch_kernel<1, kShared>), dim3(G), dim3(64), 0, st, ch, ba); break;
+    case 2: hipLaunchKernelGGL((topo_batch_kernel<2, kShared>), dim3(G), dim3(128), 0, st, ch, ba); break;
+    case 4: hipLaunchKernelGGL((topo_batch_kernel<4, kShared>), dim3(G), dim3(256), 0, st, ch, ba); break;
+    case 8: hipLaunchKernelGGL((topo_batch_kernel<8, kShared>), dim3(G), dim3(512), 0, st, ch, ba); break;
+    case 16:
+      if (d_chunks)
+        hipLaunchKernelGGL((topo_batch_kernel<16, kChunks>), dim3(G), dim3(1024), 0, st, ch, ba);
+      else
+        hipLaunchKernelGGL((topo_batch_kernel<16, kShared>), dim3(G), dim3(1024), 0, st, ch, ba);
+      break;
     default:
       set_error("unsupported waves per workgroup %d (1,2,4,8,16)", S);
       return CPET_ERR_ARG;

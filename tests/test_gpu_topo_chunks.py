@@ -112,3 +112,32 @@ def test_asked_for_workgroups_are_bounded(gpu_ctx):
     finally:
         gpu_ctx.set_tuning(2, 0, 0)
     assert torch.equal(got.view(torch.int64), want.view(torch.int64))
+
+
+# both sides of the lines between the forms of the 16-wave kernel: one group of charges a
+# slice, too few records or too many streamlines for the chunk-lane form, two workgroups a CU
+@pytest.mark.parametrize("N,L,G", [(64, 300, 0), (65, 300, 0), (149, 200, 0), (150, 200, 0),
+                                   (299, 200, 0), (300, 200, 0), (460, 30000, 0),
+                                   (470, 30000, 0), (700, 20000, 300)])
+def test_forms_are_equal(gpu_ctx, N, L, G):
+    from pycpet_amd import batch, ops
+
+    x, q, st, it = _frame(N, L, seed=N + L)
+    it = np.minimum(it, 6)
+    mu = np.random.default_rng(N).standard_normal((N, 3)).astype(np.float32)
+    frames = [{"x": x[k:], "q": q[k:], "starts": st[k::2], "n_iter": it[k::2], "h": 0.01,
+               "dims": DIMS} for k in (0, 1)]
+    try:
+        runs = []
+        for shape in ((16, G), (1, 0)):
+            for kind in (2, 3):
+                gpu_ctx.set_tuning(kind, *shape)
+            runs.append([ops.topo(st, it, 0.01, DIMS, x, q, ctx=gpu_ctx),
+                         ops.topo(st, it, 0.01, DIMS, x, q, integrator="rk4", ctx=gpu_ctx),
+                         ops.topo_dipole(st, it, 0.01, DIMS, x, mu, ctx=gpu_ctx),
+                         *batch.batch_topo(frames, ctx=gpu_ctx)])
+    finally:
+        for kind in (2, 3):
+            gpu_ctx.set_tuning(kind, 0, 0)
+    for a, b in zip(*runs):
+        _equal(a, b)
