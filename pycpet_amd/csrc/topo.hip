@@ -2041,13 +2041,21 @@ int topo_batch_run(cpet_ctx* ctx, int F, const int32_t* n_starts, const float* s
   // With the chunk-lane form a workgroup need not fill its 64 slots, and where
   // the batch is short of streamlines fewer slots let more workgroups share a
   // frame: four assignments per workgroup, as long as the slots give each wave
-  // a task (see topo_run).  Two frames of 10,206 streamlines, 8,000 charges in
-  // the mean: 32 -> 26 ms with 20 slots; eight frames of 10,648: 173 ms with
-  // 64, 182 with 48.
+  // a task (see topo_run).  Two frames of 10,000 streamlines, 8,000 charges in
+  // the mean: 90 ms with 64 slots, 66 with 20.  Fewer slots also cost rounds, each with
+  // its drain and, in the chunk-lane form, a fixed part that weighs more the fewer
+  // chunk groups there are.  With up to three groups 64 slots are better once they
+  // take all streamlines in a round or two (two frames of 9,931, 1,290 charges 13.9
+  // ms, 18.2 with 32; four of 10,000, 1,500 charges 28.6, 37.3 with 40; but six of
+  // 2,577, 1,097 charges 4.7, 4.4), with more from three rounds on (six of 7,915,
+  // 10,750 charges 46.0, 46.6 with 48; but two of 15,289, 5,300 charges 88, 73).
   int slots = 64;
   if (d_chunks && !want_far) {
-    const int want = std::max((int)(Lt / (4LL * G0)), 64 / chunk_groups(chg_off[F] / F));
-    slots = std::max(4, std::min(64, (want + 3) / 4 * 4));
+    const int groups = chunk_groups(chg_off[F] / F);
+    if (Lt < (groups <= 3 ? 62LL : 176LL) * G0) {
+      const int want = std::max((int)(Lt / (4LL * G0)), 64 / groups);
+      slots = std::max(4, std::min(64, (want + 3) / 4 * 4));
+    }
   }
   // Assignments: frames by decreasing work, one entry per A streamlines.
   // A workgroup that takes an assignment runs its 64 slots on that frame
