@@ -26,6 +26,13 @@ struct FarGrid {
 constexpr int kFarMinAxis = 8;
 constexpr double kFarMinPairs = 5e7;
 constexpr double kFarMinPairsBatch = 2e7;
+// Smaller frames of a batch that has more pairs in such frames than the one-launch
+// path takes at a time (kSmallMaxPairs).  A frame costs its 1,728 nodes instead of its
+// points, and the weights of its axes whatever its charges: 256 frames, E, kernels
+// alone, direct -> here: 21^3 x 2,000 2,054 -> 866 us, 21^3 x 250 257 -> 175, 15^3 x
+// 1,000 442 -> 410, 15^3 x 250 129 -> 149, 13^3 x 1,000 296 -> 404; 31^3 x 60 216 -> 455.
+constexpr long long kFarMinPointsMany = 3000;
+constexpr int kFarMinChargesMany = 192;
 
 // Whether an nx x ny x nz grid of npad (padded) charges takes the
 // interpolating path, from min_pairs (points x charges) on.

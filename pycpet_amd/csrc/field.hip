@@ -1017,7 +1017,6 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   // (smallfield.hip); the others stay direct
   std::vector<FarGrid> grids;
   std::vector<int> fars, smalls, direct;
-  long long small_pts = 0;
   const bool may_far = mode == kModeAuto && !(flags & CPET_F_OUT_F64) && ctx->tune[4][0] <= 0;
   const int ch_total = chg_off.empty() ? 0 : chg_off.back();
   long long pts = 0;
@@ -1043,16 +1042,46 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
                               {ax_off[f], ax_off[f] + nx, ax_off[f] + nx + ny},
                               npad, chg_off[f], out_off[f]});
       fars.push_back(f);
-      continue;
-    }
-    const long long M = (long long)nx * ny * nz;
-    if (may_far && !(E_out && phi_out && !soften) && small_field_ok(true, M, npad)) {
+    } else if (may_far && small_field_ok(true, (long long)nx * ny * nz, npad)) {
       smalls.push_back(f);
-      small_pts += M;
-      continue;
+    } else {
+      direct.push_back(f);
     }
-    direct.push_back(f);
   }
+  // The lines of single calls are lines of launches and idle CUs.  In a batch the
+  // launches are shared and the frames fill the chip together, so small frames are
+  // judged together (see kSmallMaxPairs and small_batch_ok).
+  auto points = [&](int f) { return (long long)geo[4 * f] * geo[4 * f + 1] * geo[4 * f + 2]; };
+  auto charges = [&](int f) { return chg_off[f + 1] - chg_off[f]; };
+  auto pairs_of = [&](const std::vector<int>& v) {
+    double n = 0.0;
+    for (int f : v) n += (double)points(f) * charges(f);
+    return n;
+  };
+  if (pairs_of(smalls) > kSmallMaxPairs) {
+    std::vector<int> rest;
+    for (int f : smalls) {
+      const int* g = &geo[4 * f];
+      if (points(f) >= kFarMinPointsMany && charges(f) >= kFarMinChargesMany &&
+          far_grid_ok(g[0], g[1], g[2], charges(f), 0.0)) {
+        grids.push_back(FarGrid{{g[0], g[1], g[2]},
+                                {ax_off[f], ax_off[f] + g[0], ax_off[f] + g[0] + g[1]},
+                                charges(f), chg_off[f], out_off[f]});
+        fars.push_back(f);
+      } else {
+        rest.push_back(f);
+      }
+    }
+    smalls.swap(rest);
+  }
+  int most = 0;
+  for (int f : smalls) most = std::max(most, charges(f));
+  if (!small_batch_ok(pairs_of(smalls), most, phi_out != nullptr)) {
+    direct.insert(direct.end(), smalls.begin(), smalls.end());
+    smalls.clear();
+  }
+  long long small_pts = 0;
+  for (int f : smalls) small_pts += points(f);
   std::shared_ptr<const FarPlan> plan;
   if (!fars.empty() && !(plan = far_grid_plan(ctx, grids, E_out != nullptr, phi_out != nullptr)))
     direct.insert(direct.end(), fars.begin(), fars.end());
@@ -1066,8 +1095,7 @@ int field_batch_launch(cpet_ctx* ctx, int F, const int32_t* geo3, const float* a
   const int nblk = (int)(blk.size() / 2);
   const int P = small_field_points(ctx, small_pts);
   for (int f : smalls) {
-    const long long M = (long long)geo[4 * f] * geo[4 * f + 1] * geo[4 * f + 2];
-    for (int b = 0; b < (M + P - 1) / P; ++b) {
+    for (int b = 0; b < (points(f) + P - 1) / P; ++b) {
       blk.push_back(f);
       blk.push_back(b);
     }

@@ -18,6 +18,14 @@ constexpr long long kSmallFewPoints = 4096;
 // (default precision, float32 results).
 bool small_field_ok(bool grid, long long M, int N);
 
+// Whether the small grids of a batch, of so many pairs together and at most so many
+// charges each, take this path.  It does 1.1e12 pairs/s, the direct batch kernel
+// 2.5e12 once it has enough workgroups, but a wave of that one goes through all
+// charges of its frame: 90 ns a charge at least.  256 frames of 10^3 points, here and
+// direct, us: E of 1,000 charges 238, 150, of 64 of them 65, 119; phi 171, 164 and 49, 127;
+// 21^3 x 2,000, E, 8 frames 142, 201, 64 frames 973, 516.
+bool small_batch_ok(double pairs, int most_charges, bool phi);
+
 // Float32 E and / or phi (null: not wanted; both only softened) of charges
 // x (N,3), q (N) at the points of a grid (ax, ay, az) or at pts (M,3), all on
 // the device, queued on the context's stream.

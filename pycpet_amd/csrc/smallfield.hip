@@ -181,6 +181,10 @@ bool small_field_ok(bool grid, long long M, int N) {
   return pairs <= (M <= kSmallFewPoints ? 4 : 2) * kSmallMaxPairs;
 }
 
+bool small_batch_ok(double pairs, int most_charges, bool phi) {
+  return pairs <= (phi ? 2.5e5 : 1.3e5) * most_charges;
+}
+
 // As many points per workgroup as leave about three workgroups per CU.
 int small_field_points(const cpet_ctx* ctx, long long M) {
   const long long most = 3LL * ctx->num_cus;

@@ -118,3 +118,53 @@ def test_batch(gpu_ctx, oracle_mod):
         for f, (E, phi) in zip(frames, batch.batch_volume(frames, ctx=gpu_ctx, **kw)):
             pts = np.stack(np.meshgrid(*f["axes"], indexing="ij"), -1).reshape(-1, 3)
             _check(pts, f["x"], f["q"], E, phi, oracle_mod)
+
+
+@pytest.mark.parametrize("kw", [{}, {"want_E": False, "want_phi": True}, {"want_phi": True}],
+                         ids=["E", "phi", "both"])
+def test_small_frames_are_judged_together(gpu_ctx, oracle_mod, kw):
+    """Small frames of a batch: few take the FP64 pair terms; of many, the larger grids are
+    interpolated and the smallest, and those with few charges, take the direct batch kernel, bit
+    for bit the one asked for by tuning.  refined_points() tells the three apart (all points,
+    none, those with cancellation)."""
+    from pycpet_amd import batch
+
+    def frame(n, N, seed):
+        rng = np.random.default_rng(seed)
+        axes = [np.linspace(-0.1 * (n - 1), 0.1 * (n - 1), n).astype(np.float32)] * 3
+        return {"axes": axes, "x": rng.uniform(-15, 15, (N, 3)).astype(np.float32),
+                "q": rng.normal(0, 0.4, N).astype(np.float32)}
+
+    E = kw.get("want_E", True)
+    few = [frame(9, 1000, k) for k in range(20)]
+    batch.batch_volume(few, ctx=gpu_ctx, **kw)
+    assert gpu_ctx.refined_points() == (20 * 729 if E else 0)
+
+    tiny = [frame(9, 1000, k) for k in range(400)] + [frame(16, 60, k) for k in range(5)]
+    got = batch.batch_volume(tiny, ctx=gpu_ctx, **kw)
+    assert gpu_ctx.refined_points() < (400 * 729 + 5 * 4096) / 2
+    gpu_ctx.set_tuning(4, 2, 0)
+    try:
+        want = batch.batch_volume(tiny, ctx=gpu_ctx, **kw)
+    finally:
+        gpu_ctx.set_tuning(4, 0, 0)
+    for a, b in zip(got, want):
+        for u, v in zip(a, b):
+            if u is not None:
+                np.testing.assert_array_equal(u, v)
+
+    mixed = [frame(21, 2000, k) for k in range(4)] + [frame(9, 700, 9), frame(16, 191, 10),
+                                                      frame(15, 200, 11)]
+    got = batch.batch_volume(mixed, ctx=gpu_ctx, **kw)
+    assert gpu_ctx.refined_points() == (729 if E else 0)  # 16^3 x 191 has 192 padded charges
+    for f, (e, phi) in zip(mixed, got):
+        pts = np.stack(np.meshgrid(*f["axes"], indexing="ij"), -1).reshape(-1, 3)
+        at = np.unique(np.linspace(0, len(pts) - 1, 80).astype(int))
+        pts, e, phi = pts[at], None if e is None else e[at], None if phi is None else phi[at]
+        E64, p64 = oracle_mod.field_f64(pts, f["x"], f["q"], want_phi=True)
+        r2 = ((pts[:, None].astype(np.float64) - f["x"][None]) ** 2).sum(2)
+        for u, v, mag, miss in ((e, E64, r2, 1e-9), (phi, p64, np.sqrt(r2), 1e-10)):
+            if u is not None:  # the interpolation's bounds: see test_gpu_fargrid.py
+                A = K * (np.abs(f["q"].astype(np.float64)) / mag).sum(1)
+                err = np.abs(u - v).reshape(len(pts), -1).max(1)
+                assert (err <= 2.0**-24 * np.abs(v).reshape(len(pts), -1).max(1) + miss * A).all()
