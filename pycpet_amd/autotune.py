@@ -1,9 +1,8 @@
 """Autotuner for the launch shapes of the field and streamline kernels.
 
 For a workload shape it times each candidate configuration of the runtime
-knobs (cpet_set_tuning) with HIP events on the kernel's stream, keeps the
-fastest, and caches the choice per shape bucket in a JSON file so later
-runs apply it without searching:
+knobs (cpet_set_tuning), keeps the fastest, and caches the choice per shape
+bucket in a JSON file so later runs apply it without searching:
 
   grid field     kind 0: points per lane along z (1,2,3,4,6,8) x charge splits
   streamlines    kind 2: waves per workgroup (charge slices) x workgroups
@@ -11,8 +10,13 @@ runs apply it without searching:
   batch volume   kind 4: points per lane (1,2,4)
 
 Buckets are powers of two of the charge count and of the point / streamline
-count, so frames of similar size share a choice.  Grid candidates compute the
-same per-pair arithmetic (charge splits regroup FP64 partial sums).
+count, so frames of similar size share a choice.  Streamline candidates differ
+in one kernel, which is timed with HIP events on its stream.  Grid candidates
+differ in their path: the library's own choice is one launch, or the
+interpolating ones, where a points-per-lane count asks for the direct kernel
+with its packing, near test, split sums and recompute, so whole calls are timed.
+Among the direct grid candidates the per-pair arithmetic is the same (charge
+splits regroup FP64 partial sums).
 Streamline candidates with 1 or 16 waves per workgroup give the same results
 bit for bit (the one wave walks the 16 waves' charge slices in order); 2, 4
 and 8 waves slice the charges differently, and agree to FP32 rounding.
@@ -22,6 +26,7 @@ from __future__ import annotations
 import json
 import math
 import os
+import time
 from pathlib import Path
 from typing import Callable, Dict, Iterable, Optional, Tuple
 
@@ -55,11 +60,21 @@ def save_cache(cache: Dict[str, list], path: Path = CACHE) -> None:
     os.replace(tmp, p)
 
 
+def _grid_key(kind: int, n_charges: int, n_work: int) -> str:
+    """The cache key of grid shapes chosen by whole calls.  Entries without the
+    suffix were chosen among direct kernels, or by the time of one kernel, and
+    would keep the library from its other paths."""
+    return key(kind, n_charges, n_work) + ":call"
+
+
 def sweep(ctx: nat.Context, kind: int, candidates: Iterable[Tuple[int, int]],
-          run: Callable[[], None], phase: int, repeats: int = 2) -> Tuple[Tuple[int, int], dict]:
+          run: Callable[[], None], phase: Optional[int],
+          repeats: int = 2) -> Tuple[Tuple[int, int], dict]:
     """Times run() for each (a, b) candidate; returns the best and all times
-    (ms of the kernel phase `phase` reported by cpet_ctx_phase_times)."""
-    ctx.set_profiling(True)
+    (ms of the kernel phase `phase` reported by cpet_ctx_phase_times, or, for
+    None, of the whole call up to the end of its work on the stream)."""
+    if phase is not None:
+        ctx.set_profiling(True)
     times = {}
     for a, b in candidates:
         ctx.set_tuning(kind, a, b)
@@ -67,8 +82,15 @@ def sweep(ctx: nat.Context, kind: int, candidates: Iterable[Tuple[int, int]],
             run()  # warm-up (code object load, scratch growth)
             ms = []
             for _ in range(repeats):
+                if phase is None:
+                    ctx.sync()
+                t0 = time.perf_counter()
                 run()
-                ms.append(ctx.phase_times(4)[phase])
+                if phase is None:
+                    ctx.sync()
+                    ms.append((time.perf_counter() - t0) * 1e3)
+                else:
+                    ms.append(ctx.phase_times(4)[phase])
             times[(a, b)] = float(np.median(ms))
         except nat.CpetError:
             continue
@@ -104,7 +126,7 @@ def tune_grid(ctx: nat.Context, axes, x, q, *, want_phi=False, cache: Optional[d
 
     n = int(np.prod(q.shape))
     m = int(np.prod([len(a) for a in axes]))
-    k = key(0, n, m)
+    k = _grid_key(0, n, m)
     if cache is not None and k in cache:
         a, b = cache[k]
         ctx.set_tuning(0, a, b)
@@ -112,7 +134,8 @@ def tune_grid(ctx: nat.Context, axes, x, q, *, want_phi=False, cache: Optional[d
     # (0, 0): the library's own choice, which interpolates large grids
     cands = [(0, 0)] + [(kk, s) for kk in ks for s in splits]
     best, _ = sweep(ctx, 0, cands,
-                    lambda: ops.field_grid(*axes, x, q, want_phi=want_phi, ctx=ctx), phase=0)
+                    lambda: ops.field_grid(*axes, x, q, want_phi=want_phi, ctx=ctx), phase=None,
+                    repeats=5)
     if cache is not None:
         cache[k] = list(best)
     ctx.set_tuning(0, *best)
@@ -148,14 +171,14 @@ def tune_batch_volume(ctx: nat.Context, frames, *, cache: Optional[dict] = None,
 
     n = int(np.mean([int(np.prod(f["q"].shape)) for f in frames]))
     m = int(sum(int(np.prod([len(a) for a in f["axes"]])) for f in frames))
-    k = key(4, n, m)
+    k = _grid_key(4, n, m)
     if cache is not None and k in cache:
         a, b = cache[k]
         ctx.set_tuning(4, a, b)
         return a, b
     # (0, 0): the library's own choice, which interpolates large grids
     best, _ = sweep(ctx, 4, [(0, 0)] + [(kk, 0) for kk in ks],
-                    lambda: B.batch_volume(frames, ctx=ctx), phase=0)
+                    lambda: B.batch_volume(frames, ctx=ctx), phase=None, repeats=5)
     if cache is not None:
         cache[k] = list(best)
     ctx.set_tuning(4, *best)

@@ -79,3 +79,45 @@ def test_topo_candidates_include_one_wave(monkeypatch):
         assert seen[kind][0] == (1, 0)
         assert (16, 0) in seen[kind] and len(seen[kind]) == 13
     assert ctx.calls[-1] == (3, 1, 0)  # the chosen shape is applied
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_grid_shapes_are_chosen_by_whole_calls(monkeypatch, batched):
+    """Grid candidates take different paths: the one whose first phase is shortest need not be
+    the call that is over first, and a choice that an earlier build made among direct kernels is
+    not taken over."""
+    import time
+
+    import numpy as np
+
+    from pycpet_amd import batch, ops
+
+    kind = 4 if batched else 0
+    ctx = _Ctx({})
+    ctx.times = {(0, 0): 5.0, (2, 0): 1.0, (4, 0): 2.0}     # ms of the first phase
+    wall = {(0, 0): 2e-3, (2, 0): 8e-3, (4, 0): 6e-3}       # s of the call
+    pending = []
+
+    def call(*args, **kw):
+        pending.append(wall[ctx.cur])
+
+    def sync():
+        while pending:
+            time.sleep(pending.pop())
+
+    ctx.sync = sync
+    monkeypatch.setattr(ops, "field_grid", call)
+    monkeypatch.setattr(batch, "batch_volume", call)
+    axes, x, q = [np.zeros(21, np.float32)] * 3, np.zeros((300, 3), np.float32), np.zeros(300)
+    cache = {AT.key(kind, 300, 21 ** 3): [2, 0]}
+    if batched:
+        best = AT.tune_batch_volume(ctx, [{"axes": axes, "x": x, "q": q}], cache=cache, ks=(2, 4))
+    else:
+        best = AT.tune_grid(ctx, axes, x, q, cache=cache, ks=(2, 4))
+    assert tuple(best) == (0, 0) and ctx.calls[-1] == (kind, 0, 0)
+    assert [0, 0] in cache.values() and len(cache) == 2
+    calls = len(ctx.calls)
+    ctx.times = None  # the second time the choice comes from the cache
+    again = (AT.tune_batch_volume(ctx, [{"axes": axes, "x": x, "q": q}], cache=cache, ks=(2, 4))
+             if batched else AT.tune_grid(ctx, axes, x, q, cache=cache, ks=(2, 4)))
+    assert tuple(again) == (0, 0) and len(ctx.calls) == calls + 1
