@@ -236,3 +236,32 @@ def test_batch_order_within_and_across_frames(gpu_ctx):
             np.testing.assert_array_equal(r.feats, a.feats)
             np.testing.assert_array_equal(r.steps, a.steps)
             np.testing.assert_array_equal(r.exited, a.exited)
+
+
+@pytest.mark.parametrize("out_f64", [False, True])
+def test_batch_volume_recompute_on_the_direct_kernel(gpu_ctx, oracle_mod, out_f64):
+    """The batched FP32 tiles with their check (small frames take them when a launch shape is
+    asked for): the points recomputed lie between those 10 % above and below the check's line,
+    and every point meets the 1e-5 metric."""
+    from pycpet_amd import batch
+
+    frames = [f for f in _small_frames(12) if f["kind"] == "volume"]
+    gpu_ctx.set_tuning(4, 2, 0)
+    try:
+        outs = batch.batch_volume(frames, out_f64=out_f64, ctx=gpu_ctx)
+        refined = gpu_ctx.refined_points()
+    finally:
+        gpu_ctx.set_tuning(4, 0, 0)
+    flagged = sure = total = 0
+    for f, (E, _) in zip(frames, outs):
+        pts = np.stack(np.meshgrid(*f["axes"], indexing="ij"), -1).reshape(-1, 3)
+        E64, _ = oracle_mod.field_f64(pts, f["x"], f["q"])
+        nE = np.linalg.norm(E64, axis=1)
+        d = pts[:, None].astype(np.float64) - f["x"][None].astype(np.float64)
+        A = 14.3996451 * (np.abs(f["q"].astype(np.float64)) / (d ** 2).sum(2)).sum(1)
+        flagged += (2.0 ** -24 * A >= 1.1 * 4e-6 * nE).sum()
+        sure += (2.0 ** -24 * A <= 0.9 * 4e-6 * nE).sum()
+        total += len(pts)
+        err = np.linalg.norm(E - E64, axis=1) / np.maximum(nE, 1e-3 * np.sqrt(np.mean(nE ** 2)))
+        assert err.max() <= 1e-5
+    assert 0 < flagged <= refined <= total - sure < total

@@ -403,3 +403,53 @@ def test_auto_precision_adversarial(gpu_ctx, oracle_mod, name):
     assert sure.any() or refined == pts.shape[0]  # a shell cancels everywhere: all refined
     assert (err[sure] <= 1e-5 * nE[sure]).all()
     assert rel_err(E, E64)[0] <= TOL
+
+
+def _check_recompute(pts, x, q, E, refined, oracle_mod):
+    """E within the auto mode's bounds, and as many points recomputed as its check's line allows:
+    all whose estimate u A / |E| is 10 % above 4e-6, none that is 10 % below."""
+    E64, _ = oracle_mod.field_f64(pts, x, q)
+    nE = np.linalg.norm(E64, axis=1)
+    err = np.linalg.norm(E - E64, axis=1)
+    A = np.empty(len(pts))
+    for a in range(0, len(pts), 2000):
+        d = pts[a:a + 2000, None, :].astype(np.float64) - x[None].astype(np.float64)
+        A[a:a + 2000] = 14.3996451 * (np.abs(q.astype(np.float64))[None] / (d ** 2).sum(2)).sum(1)
+    sure = 2.0 ** -24 * A <= 0.9 * 4e-6 * nE
+    flagged = 2.0 ** -24 * A >= 1.1 * 4e-6 * nE
+    print(f"refined {refined} of {len(pts)}, flagged {flagged.sum()}, sure {sure.sum()}", flush=True)
+    assert flagged.sum() <= refined <= len(pts) - sure.sum()
+    assert (err[sure] <= 1e-5 * nE[sure]).all()
+    assert rel_err(E, E64)[0] <= TOL
+
+
+@pytest.mark.parametrize("out_f64", [False, True])
+@pytest.mark.parametrize("name", ["rocksalt", "shell", "mirror1", "mirror16", "clustered"])
+def test_auto_precision_adversarial_direct(gpu_ctx, oracle_mod, name, out_f64):
+    """The layouts of test_auto_precision_adversarial on the FP32 tiles with their check, which
+    small float32 grids take when a launch shape is asked for."""
+    from pycpet_amd import ops
+
+    axes, x, q = _adversarial(name)
+    gpu_ctx.set_tuning(0, 2, 0)
+    try:
+        E, _ = ops.field_grid(*axes, x, q, out_f64=out_f64, ctx=gpu_ctx)
+        refined = gpu_ctx.refined_points()
+    finally:
+        gpu_ctx.set_tuning(0, 0, 0)
+    _check_recompute(mesh(axes), x, q, E, refined, oracle_mod)
+
+
+def test_default_grids_on_the_direct_kernel(gpu_ctx, oracle_mod):
+    """A float32 grid too large for the FP64 pair terms and, with an axis of five values, not
+    interpolated: the direct kernel by default, some points recomputed and others not."""
+    from pycpet_amd import ops
+
+    x, q, _ = _cancelling_frame()
+    axes = (np.linspace(-0.5, 0.5, 5).astype(np.float32),
+            np.linspace(-0.3, 0.4, 130).astype(np.float32),
+            np.linspace(-0.5, 0.5, 110).astype(np.float32))
+    E, _ = ops.field_grid(*axes, x, q, ctx=gpu_ctx)
+    refined = gpu_ctx.refined_points()
+    assert 0 < refined < 5 * 130 * 110
+    _check_recompute(mesh(axes), x, q, E, refined, oracle_mod)
