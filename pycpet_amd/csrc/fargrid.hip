@@ -10,7 +10,8 @@
 // path are summed directly at the point.  All sums, nodes and interpolation
 // are FP64 (the pair terms as in the "mixed" precision: FP64 displacement and
 // r^2, FP32 rsq seed, FP64 correction), so nothing needs the FP32 error check
-// and recompute of the direct grid kernel.
+// and recompute of the direct grid kernel; points where E nearly cancels are
+// summed again without interpolation, in far_eval (see kCancel).
 //
 // Far means that along every axis the nearest singularity of the charge's
 // field, seen from any point of the cell, lies outside the Bernstein ellipse
@@ -33,7 +34,7 @@
 // Every list and sum has a fixed order: results are reproducible bit for bit.
 
 #include <algorithm>
-#include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "cpet_internal.h"
@@ -75,6 +76,14 @@ constexpr float kInvS2 = 1.0f / (kSigma * kSigma);
 constexpr float kInvS21 = 1.0f / (kSigma * kSigma - 1.0f);
 constexpr float kMinGap2 = 1e-4f;   // 0.01 A: far charges never reach the r^2 floor
 constexpr float kMaxCoord = 1e6f;   // beyond (or not finite): summed directly
+// A point whose E is below this share of S = sum |q| / gap^2 over the charges
+// interpolated for its leaf (gap: from the cell at whose nodes) is summed directly: what
+// the interpolation misses, some 1e-12 S where charges are placed so that their
+// misses add up (a shell of equal charges, mirrored ones), would be more than E's
+// rounding there (2-norm error of a shell's E 1.4e-7, with this 2.5e-8).  Hardly a
+// point of other frames: 1 in 1e8 at random.  S costs the classification 0.2 us (12k
+// x 61 x 47 x 38) to 1.1 us (30k x 101^3), the test 0.2 us of far_eval.
+constexpr double kCancel = 2e-5;
 
 // cos((2k + 1) pi / 24) and (-1)^k sin((2k + 1) pi / 24): the Chebyshev nodes
 // of the first kind and their barycentric weights.
@@ -106,7 +115,8 @@ struct FarFrame {
   long long lag0[3];   // per axis: level x axis value x kP weights
   long long tr0[3];    // per axis: leaf part x ancestor level x kP x kP
   long long mask0;     // (cells + leaves) x nseg: far masks, then the leaves' near masks
-  long long near0;     // per leaf: number of near charges, then their numbers (64 nseg)
+  long long mag0;      // cells x nseg: sum |q| / gap^2 of a segment's charges far from the cell
+  long long near0;     // per leaf: number of near charges, S, then their numbers (64 nseg)
   int leaf0;           // the launch's first leaf (see Group::range)
   long long out0;      // first output point
   long long ax0[3];    // first value of each axis
@@ -123,6 +133,7 @@ struct FarArgs {
   double* geo;
   double* lag;
   unsigned long long* mask;
+  float* mag;
   int* near;
   void* e;
   void* phi;
@@ -276,8 +287,26 @@ __device__ void axis_tables(const FarArgs& A, Frame& f, int axis, int share, con
   }
 }
 
-// Whether a charge is far from the cell with centre m and half widths a.
-__device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], const float (&a)[3]) {
+// Sum of v over the wave, in lane 63.
+__device__ __forceinline__ float wave_sum63(float v) {
+  auto add = [&](auto ctrl, auto rows) __attribute__((always_inline)) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value,
+                                                    decltype(rows)::value, 0xf, false));
+  };
+  using std::integral_constant;
+  add(integral_constant<int, 0x111>(), integral_constant<int, 0xf>());  // row_shr:1, 2, 4, 8
+  add(integral_constant<int, 0x112>(), integral_constant<int, 0xf>());
+  add(integral_constant<int, 0x114>(), integral_constant<int, 0xf>());
+  add(integral_constant<int, 0x118>(), integral_constant<int, 0xf>());
+  add(integral_constant<int, 0x142>(), integral_constant<int, 0xa>());  // row_bcast:15, 31
+  add(integral_constant<int, 0x143>(), integral_constant<int, 0xc>());
+  return v;
+}
+
+// Whether a charge is far from the cell with centre m and half widths a; gap2: its
+// squared distance from the cell.
+__device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], const float (&a)[3],
+                                         float& gap2) {
   const float x[3] = {c.x, c.y, c.z};
   float d2[3], g2[3];
   bool ok = fabsf(c.w) < 1e30f;
@@ -289,7 +318,8 @@ __device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], c
     d2[i] = d * d;
     g2[i] = gap * gap;
   }
-  ok = ok && g2[0] + g2[1] + g2[2] >= kMinGap2;
+  gap2 = g2[0] + g2[1] + g2[2];
+  ok = ok && gap2 >= kMinGap2;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
     ok = ok && fmaf(d2[i], kInvS2, (g2[(i + 1) % 3] + g2[(i + 2) % 3]) * kInvS21) >= a[i] * a[i];
@@ -303,6 +333,7 @@ __device__ __forceinline__ bool far_from(const float4& c, const float (&m)[3], c
 // exactly one mask of every leaf's path.  A cell whose parent is near none
 // of the wave's charges is skipped.  Padding is in no mask.  The frame's last
 // workgroups make the tables, kTableBlocks those of one axis.
+template <bool E>
 __global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) {
   extern __shared__ char dyn[];
   Frame& f = frame_of_block(&FarFrame::class_blk0, blockIdx.x);
@@ -313,6 +344,7 @@ __global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) 
   double* sa = sm + 3 * kGeoPerAxis;
   unsigned long long* far = (unsigned long long*)(sa + 3 * kGeoPerAxis);  // cells
   unsigned long long* near = far + f.cells;                               // cells
+  float* mag = (float*)(near + f.cells);                                  // cells
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int only = b < f.nseg ? -1 : (b - f.nseg) / kTableBlocks;  // table workgroups: their axis
   float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -347,6 +379,7 @@ __global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) 
       const unsigned long long pm =
           level ? near[parent0 + ancestor(f, level - 1, level, t)] : all;
       unsigned long long mf = 0ull;
+      [[maybe_unused]] float s = 0.f;
       if (pm) {
         float m[3], a[3];
 #pragma unroll
@@ -355,11 +388,15 @@ __global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) 
           m[i] = (float)sm[e];
           a[i] = (float)sa[e];
         }
-        mf = __ballot(far_from(c, m, a)) & pm;
+        float gap2;
+        const bool mine = far_from(c, m, a, gap2) && ((pm >> lane) & 1);
+        mf = __ballot(mine);
+        if constexpr (E) s = wave_sum63(mine ? fabsf(c.w) * __builtin_amdgcn_rcpf(gap2) : 0.f);
       }
-      if (lane == 0) {
+      if (lane == 63) {
         far[cell0 + k] = mf;
         near[cell0 + k] = pm & ~mf;
+        if constexpr (E) mag[cell0 + k] = s;
       }
     }
     __syncthreads();
@@ -368,10 +405,17 @@ __global__ __launch_bounds__(kClassThreads) void far_classify_kernel(FarArgs A) 
   }
   const int leaves = cell0 - parent0;
   unsigned long long* out = A.mask + f.mask0 + b;
-  for (int k = threadIdx.x; k < f.cells; k += kClassThreads) out[(long long)k * f.nseg] = far[k];
+  for (int k = threadIdx.x; k < f.cells; k += kClassThreads) {
+    out[(long long)k * f.nseg] = far[k];
+    if constexpr (E) A.mag[f.mag0 + (long long)k * f.nseg + b] = mag[k];
+  }
   for (int k = threadIdx.x; k < leaves; k += kClassThreads)
     out[(long long)(f.cells + k) * f.nseg] = near[parent0 + k];
 }
+
+constexpr int kNearHead = 2;  // number of near charges, S
+
+__host__ __device__ inline long long near_stride(int nseg) { return kNearHead + 64LL * nseg; }
 
 // ---- charges of a mask list ------------------------------------------------
 
@@ -474,9 +518,23 @@ __global__ __launch_bounds__(kNodeThreads, 6) void far_nodes_kernel(FarArgs A) {
     const unsigned long long* __restrict__ mask =
         A.mask + f.mask0 + (long long)(f.cells + f.leaf0 + b) * f.nseg;
     const int total = list_prefix<kNodeThreads>(mask, f.nseg, off, tmp);
-    int* out = A.near + f.near0 + (long long)b * (64 * f.nseg + 1);
+    int* out = A.near + f.near0 + (long long)b * near_stride(f.nseg);
+    for (int r = tid; r < total; r += kNodeThreads)
+      out[kNearHead + r] = list_charge(mask, f.nseg, off, r);
     if (tid == 0) out[0] = total;
-    for (int r = tid; r < total; r += kNodeThreads) out[1 + r] = list_charge(mask, f.nseg, off, r);
+    if (E && tid >= kNodeThreads - 64) {  // S: the cells of the leaf's path, in a fixed order
+      int t[3];
+      cell_parts(f, f.levels - 1, f.leaf0 + b, t);
+      double s = 0.0;
+      for (int k = 0, first = 0; k < f.levels; first += cells_at(f, k++)) {
+        const float* __restrict__ mag =
+            A.mag + f.mag0 + (long long)(first + ancestor(f, k, f.levels - 1, t)) * f.nseg;
+        for (int i = tid & 63; i < f.nseg; i += 64) s += (double)mag[i];
+      }
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d);
+      if ((tid & 63) == 0) out[1] = __float_as_int((float)s);
+    }
     return;
   }
   const int third = b % kThirds, slot = b / kThirds;
@@ -644,8 +702,11 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
     double wt[kPC * kP * kP];
     double4 list[kNearLds];
   } u;
+  __shared__ unsigned short redo[E ? kPlanes * kLeafMax * kLeafMax : 1];  // points to sum directly
+  __shared__ int redos;
   double* const wt = u.wt;
   const int tid = threadIdx.x;
+  if (E && tid == 0) redos = 0;
   const double* __restrict__ lagy =
       A.lag + f.lag0[1] + ((long long)f.l[1] * f.n[1] + lo[1]) * kP;
   const double* __restrict__ lagz =
@@ -728,9 +789,10 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
     for (int k = 0; k < kP; ++k) s = fma(lagy[j * kP + k], w1[pc * kP * kP + k * kP + c], s);
     w2[(pc * kLeafMax + j) * kP + c] = s;
   }
-  const int* __restrict__ near = A.near + f.near0 + (long long)list * (64 * f.nseg + 1);
+  const int* __restrict__ near = A.near + f.near0 + (long long)list * near_stride(f.nseg);
   const float4* __restrict__ ch = A.ch + f.ch0;
   const int total = near[0];
+  const double least = E ? kCancel * (double)__int_as_float(near[1]) : 0.0;
   __syncthreads();
   // z, the near charges and the store
   const float* __restrict__ ax = A.ax[0] + f.ax0[0];
@@ -765,7 +827,7 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
       if (i0 == 0 || total > kNearLds) {  // a short list stays staged
         __syncthreads();
         if (tid < qn) {
-          const float4 c = ch[near[1 + q0 + tid]];
+          const float4 c = ch[near[kNearHead + q0 + tid]];
           u.list[tid] = make_double4(c.x, c.y, c.z, c.w);
         }
         __syncthreads();
@@ -799,9 +861,47 @@ __global__ __launch_bounds__(kEvalThreads, E && PHI ? 3 : 4) void far_eval_kerne
           e[0] = (float)(kCoulomb * acc[k][0]);
           e[1] = (float)(kCoulomb * acc[k][1]);
           e[2] = (float)(kCoulomb * acc[k][2]);
+          if (fma(acc[k][2], acc[k][2], fma(acc[k][1], acc[k][1], acc[k][0] * acc[k][0])) <
+              least * least)
+            redo[atomicAdd(&redos, 1)] = (unsigned short)((p * n[1] + j) * n[2] + k0 + k);
         }
         if constexpr (PHI) ((float*)A.phi)[m0 + k] = (float)(kCoulomb * acc[k][C - 1]);
       }
+  }
+  if constexpr (E) {
+    __syncthreads();
+    const int again = redos;
+    for (int i = 0; i < again; ++i) {  // the whole workgroup, charge by charge
+      const int pt = redo[i];
+      const int k = pt % n[2], j = pt / n[2] % n[1], p = pt / (n[1] * n[2]);
+      const double px = ax[x0 + p], py = ay[lo[1] + j], pz = az[lo[2] + k];
+      double e[3] = {0.0, 0.0, 0.0};
+      for (int q = tid; q < 64 * f.nseg; q += kEvalThreads) {
+        const float4 c = ch[q];
+        const double dx = px - (double)c.x, dy = py - (double)c.y, dz = pz - (double)c.z;
+        double re;
+        pair_rsqrt<SOFT, !PHI>(fma(dz, dz, fma(dy, dy, dx * dx)), rclamp, re);
+        const double w = ((double)c.w * re) * (re * re);
+        e[0] = fma(w, dx, e[0]);
+        e[1] = fma(w, dy, e[1]);
+        e[2] = fma(w, dz, e[2]);
+      }
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) e[c] += __shfl_xor(e[c], d);
+      if ((tid & 63) == 0)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) lz[(tid >> 6) * 3 + c] = e[c];
+      __syncthreads();
+      if (tid < 3) {
+        double v = 0.0;
+        for (int w = 0; w < kEvalThreads / 64; ++w) v += lz[w * 3 + tid];
+        const long long m = f.out0 + ((long long)(x0 + p) * f.n[1] + lo[1] + j) * f.n[2] + lo[2] + k;
+        ((float*)A.e)[3 * m + tid] = (float)(kCoulomb * v);
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -820,8 +920,10 @@ struct Group {
   // Leaves whose near lists are held at once, of the leaves of one frame whose lists
   // (room for every charge in each) would not fit the scratch bound; 0: all of them.
   int range = 0, leaves = 0;
-  long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, near = 0;
-  size_t bytes() const { return (size_t)(part + val + geo + lag + mask) * 8 + (size_t)near * 4; }
+  long long part = 0, val = 0, geo = 0, lag = 0, mask = 0, mag = 0, near = 0;
+  size_t bytes() const {
+    return (size_t)(part + val + geo + lag + mask) * 8 + (size_t)(mag + near) * 4;
+  }
 };
 
 template <bool E, bool PHI>
@@ -839,7 +941,7 @@ void far_launch(hipStream_t st, FarArgs A, const Group& n, bool soft) {
       hipLaunchKernelGGL((far_eval_kernel<E, PHI, false>), dim3((unsigned)blocks),
                          dim3(kEvalThreads), 0, st, A);
   };
-  hipLaunchKernelGGL(far_classify_kernel, dim3((unsigned)n.classify), dim3(kClassThreads), n.lds, st, A);
+  hipLaunchKernelGGL((far_classify_kernel<E>), dim3((unsigned)n.classify), dim3(kClassThreads), n.lds, st, A);
   nodes(n.nodes);
   if (n.reduce)
     hipLaunchKernelGGL((far_reduce_kernel<C>), dim3((unsigned)n.reduce), dim3(kRedThreads), 0, st,
@@ -928,6 +1030,7 @@ std::shared_ptr<const FarPlan> far_grid_plan(cpet_ctx* ctx, const std::vector<Fa
       f.val0 = n.val;
       f.geo0 = n.geo;
       f.mask0 = n.mask;
+      f.mag0 = n.mag;
       f.near0 = n.near;
       long long p = 0, nb = 0, rb = 0, leaves = 0;
       for (int k = 0; k < f.levels; ++k) {
@@ -949,17 +1052,18 @@ std::shared_ptr<const FarPlan> far_grid_plan(cpet_ctx* ctx, const std::vector<Fa
       with.part += p;
       with.val += (long long)f.cells * C * kNodes;
       with.mask += (f.cells + leaves) * f.nseg;
-      with.near += leaves * (64LL * f.nseg + 1);
+      with.mag += (long long)f.cells * f.nseg;
+      with.near += leaves * near_stride(f.nseg);
       with.geo += 3LL * kGeoPerAxis * 2;
       if (n.count && with.bytes() > kMaxScratch) break;
       long long lists = leaves;
       if (with.bytes() > kMaxScratch) {  // a frame alone
-        const size_t list = (64 * (size_t)f.nseg + 1) * 4;
+        const size_t list = (size_t)near_stride(f.nseg) * 4;
         const size_t rest = with.bytes() - leaves * list;
         lists = rest + list < kMaxScratch ? (long long)((kMaxScratch - rest) / list) : 1;
         with.range = (int)lists;
         with.leaves = (int)leaves;
-        with.near = lists * (64LL * f.nseg + 1);
+        with.near = lists * near_stride(f.nseg);
       }
       const int widest = (f.n[0] + (1 << f.l[0]) - 1) >> f.l[0];
       f.xblocks = (widest + kPlanes - 1) / kPlanes;
@@ -968,7 +1072,7 @@ std::shared_ptr<const FarPlan> far_grid_plan(cpet_ctx* ctx, const std::vector<Fa
       with.reduce += rb;
       with.eval += lists * f.xblocks;
       with.lds = std::max(n.lds, (size_t)((values * 4 + 15) & ~15) + 6 * kGeoPerAxis * 8 +
-                                     (size_t)f.cells * 16);
+                                     (size_t)f.cells * 20);
       ++with.count;
       n = with;
       frames.push_back(f);
@@ -1001,7 +1105,8 @@ int far_grid_run(cpet_ctx* ctx, const FarPlan& plan, const float* const (&ax)[3]
     A.geo = A.val + n.val;
     A.lag = A.geo + n.geo;
     A.mask = (unsigned long long*)(A.lag + n.lag);
-    A.near = (int*)(A.mask + n.mask);
+    A.mag = (float*)(A.mask + n.mask);
+    A.near = (int*)(A.mag + n.mag);
     A.e = e;
     A.phi = phi;
     if (n.count == 1)

@@ -358,3 +358,46 @@ def test_largest_plan(oracle_mod, n, charges):
                oracle_mod)
     del E, out
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batched", [False, True])
+@pytest.mark.parametrize("name", ["shell", "mirror"])
+def test_points_where_the_field_cancels(gpu_ctx, oracle_mod, name, batched):
+    """Layouts whose interpolation misses add up while the field itself cancels (E of 1e-6 of
+    the terms' magnitudes A and less): points below 2e-5 of it are summed directly, whose pair
+    terms are good to 1e-14, so 1e-13 A beside the rounding is allowed there."""
+    from pycpet_amd import batch, ops
+
+    rng = np.random.default_rng(4)
+    if name == "shell":  # equal charges on a sphere: E ~ 0 inside
+        k = np.arange(6000) + 0.5
+        ph, th = np.arccos(1 - 2 * k / 6000), np.pi * (1 + 5 ** 0.5) * k
+        x = 9 * np.stack([np.cos(th) * np.sin(ph), np.sin(th) * np.sin(ph), np.cos(ph)], 1)
+        q = np.full(6000, 0.3)
+    else:  # point symmetric: E = 0 at the centre
+        h = rng.uniform(-12, 12, (3000, 3))
+        h = h[(np.abs(h) > 3.5).any(1)]
+        x = np.concatenate([h, -h])
+        q = np.tile(rng.normal(0, 0.4, len(h)), 2)
+    x, q = x.astype(np.float32), q.astype(np.float32)
+    axes = [np.linspace(-2, 2, 41).astype(np.float32)] * 3
+    if batched:
+        E = batch.batch_volume([{"axes": axes, "x": x, "q": q}] * 2, ctx=gpu_ctx)[1][0]
+    else:
+        E, _ = ops.field_grid(*axes, x, q, ctx=gpu_ctx)
+    E2, _ = ops.field_grid(*axes, x, q, want_phi=True, ctx=gpu_ctx)
+    pts = _mesh(axes)
+    at = np.unique(np.concatenate([[len(pts) // 2], rng.choice(len(pts), 1500, replace=False)]))
+    pts = pts[at]
+    E64, _ = oracle_mod.field_f64(pts, x, q)
+    A = np.empty(len(pts))
+    for a in range(0, len(pts), 100):
+        d2 = ((pts[a:a + 100, None].astype(np.float64) - x[None]) ** 2).sum(2)
+        A[a:a + 100] = K * (np.abs(q) / d2).sum(1)
+    nE = np.linalg.norm(E64, axis=1)
+    low = nE <= 1e-5 * A
+    assert low[at == 41 ** 3 // 2].all() and (name == "mirror" or low.all())
+    for e in (E[at], E2[at]):
+        err = np.linalg.norm(e - E64, axis=1)
+        assert (err <= 1.1 * 2.0**-24 * nE + np.where(low, 1e-13, 1e-9) * A).all()
