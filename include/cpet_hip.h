@@ -336,6 +336,8 @@ int cpet_compact_charges(cpet_ctx *ctx, int N, const uint8_t *keep, const float 
  *   cpet_topo:          [order, propagate, epilogue(+histogram)]
  *   cpet_field_*:       [field kernel, split reduction, FP64 recompute]
  *   cpet_batch_volume:  [field kernel, FP64 recompute]
+ * (of the direct kernels; the interpolating and the one-launch path count
+ * whole in the first, so phases do not compare paths).
  * No counterpart in the reference (its timing is time.time() around calls,
  * CPET/source/calculator.py:686,706-711). */
 int cpet_ctx_set_profiling(cpet_ctx *ctx, int on);
@@ -344,8 +346,9 @@ int cpet_ctx_phase_times(cpet_ctx *ctx, float *ms, int n);
 /* Number of grid / points the last field call on this context recomputed in
  * FP64 because the auto-precision check found strong cancellation there
  * (u * sum|q|/r^2 > 4e-6 * |E|); all of them when the call was small and
- * summed everything in FP64; 0 when that call had no check (precision modes
- * other than auto, or no E requested).  Waits for the context's
+ * summed everything in FP64; 0 when that call had no such check (precision
+ * modes other than auto, no E requested, or an interpolated grid, whose own
+ * check is not counted).  Waits for the context's
  * stream.  No counterpart in the reference (its sums are FP32 throughout,
  * CPET/utils/math_module.c:405-451). */
 int cpet_ctx_refined_points(cpet_ctx *ctx, long long *n);
@@ -362,9 +365,10 @@ int cpet_ctx_refined_points(cpet_ctx *ctx, long long *n);
  *   per workgroup).  Streamline results are the same bit for bit with 16
  *   waves and with 1 wave per workgroup (the one wave walks the 16 waves'
  *   charge slices in order); 2, 4 and 8 waves split the charges
- *   differently and agree to FP32 rounding.  The default is 1 wave for a
- *   batch whose frames all have at most 128 charges and for a single frame
- *   of at most 16 charges and at least 50,000 starts, else 16. */
+ *   differently and agree to FP32 rounding.  More 16-wave workgroups than
+ *   CUs are launched only where each has 64 streamlines.  The default is 1
+ *   wave for a batch whose frames all have at most 128 charges and for a
+ *   single frame of at most 16 charges and at least 50,000 starts, else 16. */
 int cpet_set_tuning(cpet_ctx *ctx, int kind, int a, int b);
 
 /* ------------------------------------------------------ cluster step

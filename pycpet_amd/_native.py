@@ -222,7 +222,8 @@ class Context:
         return list(buf)
 
     def refined_points(self) -> int:
-        """Points the last auto-precision field call recomputed in FP64."""
+        """Points the last auto-precision field call recomputed in FP64 (all of
+        them if it was small and summed everything in FP64)."""
         n = ctypes.c_longlong(0)
         check(self.lib.cpet_ctx_refined_points(self.handle, ctypes.byref(n)), self.lib)
         return n.value

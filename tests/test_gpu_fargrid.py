@@ -325,7 +325,7 @@ def test_captured_batch_of_several_scratch_groups(gpu_ctx):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n, charges", [((217, 217, 217), 200), ((217, 218, 217), 45000)])
 def test_largest_plan(oracle_mod, n, charges):
-    """Four halvings on every axis (4,681 cells, 80 KB of LDS in the classification), with few
+    """Four halvings on every axis (4,681 cells, 100 KB of LDS in the classification), with few
     charges, and with so many that the near lists of all leaves would need 740 MB: right, and
     within 1 GiB of scratch (and the quarter that the context adds)."""
     import torch
